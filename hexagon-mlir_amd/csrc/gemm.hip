@@ -661,13 +661,14 @@ static int64_t stream_k_bytes(const KernelEntry& e, const StreamKLayout& sk) {
 
 // plan_gemm for the W8A16 GEMMs (f16 A, int8 [N, K] B): N is the B rows
 // (the SwiGLU image's), n_out the output columns.
-hxm_status plan_gemm_w8(int32_t op, bool sw, int64_t M, int64_t N, int64_t n_out, int64_t K,
+hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out, int64_t K,
                         const hxm_gemm_config* cfg, hxm_plan* p, const KernelEntry** entry) {
   *p = hxm_plan{};
   p->op = op;
   p->m = M, p->n = n_out, p->k = K;
   p->plan = HXM_PLAN_REFUSED;
   p->k_slices = 1;
+  const bool sw = epi == kEpiSwiglu;
   char why[192];
   hxm_gemm_config c;
   if (cfg && cfg->bm) {
@@ -676,13 +677,25 @@ hxm_status plan_gemm_w8(int32_t op, bool sw, int64_t M, int64_t N, int64_t n_out
   } else if (lookup_tuned(op, M, sw ? n_out : N, K, &c)) {
     p->source = HXM_SOURCE_TUNED;
   } else {
-    c = default_w8_config(M, N, sw);
+    c = skinny_fits(M, n_out, K) ? skinny_config() : default_w8_config(M, N, sw);
     p->source = HXM_SOURCE_DEFAULT;
   }
   p->config = c;
   hxm_status st = HXM_OK;
-  const KernelEntry* e = find_w8_kernel(c, sw);
-  if (!e) {
+  const bool skinny = is_skinny_config(c);
+  const KernelEntry* e = skinny ? nullptr : find_w8_kernel(c, sw);
+  if (skinny) {
+    if (!skinny_fits(M, n_out, K)) {
+      snprintf(why, sizeof(why), "the skinny kernel takes 1 to %lld rows and K > 0",
+               (long long)kSkinnyRowsMax);
+      st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_NO_KERNEL, why);
+    } else {
+      skinny_plan_w8(epi, M, n_out, p);
+      const bool full = M % 32 == 0 && n_out % 32 == 0 && K % 32 == 0;
+      p->plan = full ? HXM_PLAN_MFMA_FULL : HXM_PLAN_MFMA_TAIL;
+      p->reason = full ? HXM_REASON_SELECTED_ALIGNED : HXM_REASON_SELECTED_TAIL;
+    }
+  } else if (!e) {
     const bool plain = find_w8_kernel(c, false) != nullptr;
     snprintf(why, sizeof(why), "no compiled W8A16 GEMM%s for bm=%d bn=%d bk=%d waves=%dx%d",
              sw ? " with the SwiGLU epilogue (its wave tile is 128 wide)" : "", c.bm, c.bn,
@@ -741,7 +754,7 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
   const bool sw = epi == kEpiSwiglu;
   const KernelEntry* e = nullptr;
   hxm_plan plan;
-  hxm_status st = plan_gemm_w8(op, sw, M, N, n_out, K, cfg, &plan, &e);
+  hxm_status st = plan_gemm_w8(op, epi, M, N, n_out, K, cfg, &plan, &e);
   if (st != HXM_OK) return st;
   if ((st = require_device(nullptr)) != HXM_OK) return st;
   if (M == 0 || N == 0) return ok();
@@ -766,6 +779,10 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
   g.res_vec8 = residual && (reinterpret_cast<uintptr_t>(residual) % 16 == 0) && ((ldr * 2) % 16 == 0);
   g.vec_store = (reinterpret_cast<uintptr_t>(C) % 8 == 0) && ((ldc * 2) % 8 == 0);
   g.vec8_store = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && ((ldc * 2) % 16 == 0);
+  if (!e) {  // the plan chose the skinny kernel
+    if ((st = launch_skinny_w8(epi, g, stream)) != HXM_OK) return st;
+    return ok();
+  }
   const int wi = static_cast<int>(e - kW8Kernels);
   int64_t groups = plan.tiles;
   if (plan.config.split_k == HXM_STREAM_K) {

@@ -1303,6 +1303,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
 
 typedef void (*gemm_fn)(GemmArgs);
 
+// The skinny W8A16 matmul (gemm_skinny.hip): fills a plan's config, threads,
+// tiles and LDS; launches (g as for the tile kernels).
+void skinny_plan_w8(int epi, int64_t M, int64_t n_out, hxm_plan* p);
+hxm_status launch_skinny_w8(int epi, const GemmArgs& g, hipStream_t stream);
+
 // The compiled kernels.  Each kernel source (gemm_i8.hip, gemm_f16.hip,
 // gemm_w8.hip) is compiled kGemmParts times with HXM_PART = 0 .. kGemmParts-1
 // so the objects build in parallel: part p instantiates the configurations

@@ -91,6 +91,13 @@ hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const
                              int64_t K, int32_t out_dtype, int32_t accumulate,
                              hipStream_t stream);
 
+// The skinny W8A16 matmul (gemm_skinny.hip): the default of the W8A16 GEMMs at
+// 1 to kSkinnyRowsMax rows; a caller names it with skinny_config().
+constexpr int64_t kSkinnyRowsMax = 64;
+hxm_gemm_config skinny_config();
+bool is_skinny_config(const hxm_gemm_config& c);
+bool skinny_fits(int64_t M, int64_t N, int64_t K);
+
 }  // namespace hxm
 
 #define HXM_HIP_TRY(expr)                                                    \

@@ -403,10 +403,12 @@ hxm_status tune_core(const TuneSpec& sp, int32_t reps, hxm_gemm_config* best, ch
     if (measure(cands[i], M, N, K, &samples) != HXM_OK) continue;  // scores inf
     if (have_ref) {
       HXM_HIP_TRY(hipMemsetAsync(bad, 0, sizeof(unsigned), s));
-      // The direct-load small-output kernel and the stream-K tiles (fp32
-      // partial tiles added across workgroups) sum in another order than the
-      // staged one-workgroup tiles: checked within the float tolerance.
+      // The direct-load small-output kernel, the skinny kernel (partial sums
+      // of its waves) and the stream-K tiles (fp32 partial tiles added across
+      // workgroups) sum in another order than the staged one-workgroup tiles:
+      // checked within the float tolerance.
       if (is_small_gemm_config(cands[i]) != is_small_gemm_config(control) ||
+          is_skinny_config(cands[i]) != is_skinny_config(control) ||
           (cands[i].split_k == HXM_STREAM_K) != (control.split_k == HXM_STREAM_K))
         count_far_kernel<<<1024, 256, 0, s>>>(static_cast<const uint32_t*>(C),
                                               (ldc * out_eb) / 4, ref, M, row_words,
@@ -814,7 +816,9 @@ hxm_status hxm_tune_cache_load(const char* path, int32_t* loaded) {
     // The small-output kernel is a winner only for shapes it takes.
     const bool small_ok = (op == HXM_F16 || op == HXM_BF16) && is_small_gemm_config(c) &&
                           small_gemm_fits(ent.m, ent.n, ent.k, op);
-    if (!small_ok && !config_compiled(op, c)) continue;
+    const bool skinny_ok = (op == HXM_OP_W8A16 || op == HXM_OP_W8A16_SWIGLU) &&
+                           is_skinny_config(c) && skinny_fits(ent.m, ent.n, ent.k);
+    if (!small_ok && !skinny_ok && !config_compiled(op, c)) continue;
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[TuneKey(op, ent.m, ent.n, ent.k)] = c;
     g_tuned_reps[TuneKey(op, ent.m, ent.n, ent.k)] = ent.reps;
@@ -949,6 +953,10 @@ hxm_status hxm_tune_w8a16(int32_t op, const void* x, int64_t ldx, const int8_t* 
   sort_configs(&sp.cands);
   sp.control = default_w8_config(M, rows, sw);
   sp.canary = sp.cands.front();  // the smallest compiled tile on a 32-row slice
+  if (skinny_fits(M, N, K)) {    // what an untuned call runs
+    sp.control = skinny_config();
+    sp.cands.insert(sp.cands.begin(), sp.control);
+  }
   sp.cm = std::min<int64_t>(32, M), sp.cn = std::min<int64_t>(sw ? 64 : 32, N);
   sp.ck = std::min<int64_t>(K, 32);
   sp.run = [=](const hxm_gemm_config& c, int64_t m, int64_t n, int64_t k) {

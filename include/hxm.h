@@ -366,7 +366,11 @@ enum { HXM_OP_W8A16 = 16, HXM_OP_W8A16_SWIGLU = 17 };
  * rtol 1e-2 / atol 1e-3).  K multiple of 16, ldx multiple of 8, ldw
  * multiple of 16, x and W 16-byte aligned, and 256 rows of x and of W
  * within 2 GiB (as for hxm_matmul).  cfg: NULL = tuned winner or the
- * default tile; else one of hxm_w8a16_configs. */
+ * default; else one of hxm_w8a16_configs.  With cfg NULL and no tuned winner,
+ * 1 to 64 rows run on the skinny kernel (config {16,16,64,1,8,0,1}: the
+ * waves of a workgroup split K, partial sums added in a fixed order); the
+ * same config passed in cfg asks for it and is refused
+ * (HXM_UNSUPPORTED_SHAPE, "no-kernel") outside those limits. */
 hxm_status hxm_gemm_w8a16(const void* x, int64_t ldx, const int8_t* W,
                           int64_t ldw, const float* w_scale, void* y,
                           int64_t ldy, int64_t M, int64_t N, int64_t K,
