@@ -58,15 +58,21 @@ struct OpSum {
   }
 };
 
-// Reduces v over all 64 lanes; the result is wave-uniform.  Inside each
-// 16-lane row: xor-1, xor-2, half-mirror, mirror (every lane ends with its
-// row's total); across rows: four readlanes folded pairwise.
+// Reduces v over each 16-lane row; every lane ends with its row's total.
+// xor-1, xor-2, half-mirror, mirror.
 template <typename Op>
-__device__ __forceinline__ float wave_reduce(float v, Op op) {
+__device__ __forceinline__ float row16_reduce(float v, Op op) {
   v = op(v, dpp<kDppQuadXor1>(v));
   v = op(v, dpp<kDppQuadXor2>(v));
   v = op(v, dpp<kDppRowHalfMirror>(v));
-  v = op(v, dpp<kDppRowMirror>(v));
+  return op(v, dpp<kDppRowMirror>(v));
+}
+
+// Reduces v over all 64 lanes; the result is wave-uniform: the four 16-lane
+// totals, then four readlanes folded pairwise.
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+  v = row16_reduce(v, op);
   float a = op(readlane(v, 0), readlane(v, 16));
   float b = op(readlane(v, 32), readlane(v, 48));
   return op(a, b);

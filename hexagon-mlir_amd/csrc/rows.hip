@@ -7,14 +7,17 @@
 // lib/Conversion/LinalgToLLVM/VectorRowReducePass.cpp:10-31 (vector fold +
 // rotate butterfly) and SplitReduceGenericPass.cpp:62-93.
 //
-// Design: one wave per row, four rows per 256-thread workgroup.  A row of up to
-// 64 lanes x 16 vectors x 16 bytes is loaded ONCE into registers with 128-bit
-// coalesced loads (consecutive lanes read consecutive 16-byte chunks), reduced
-// across the wave with DPP + readlane (no LDS, no barriers) and written back
-// from registers: one HBM read and one HBM write per element.  Full rows of 8
-// vectors per lane (4096 f16) are split over two or four waves whose totals
-// meet in LDS (see row_kernel).  Longer rows use the streaming variant
-// (VPL = 0) that re-reads the row per pass.
+// Design: a row is loaded ONCE into registers with 128-bit loads (consecutive
+// lanes read consecutive 16-byte chunks), reduced across each wave with DPP +
+// readlane and across the S waves that share the row through LDS, and written
+// back from registers: one HBM read and one HBM write per element.  S grows
+// with the row: one wave up to 128 vectors of 16 bytes, then 2, 4, 8 and 16
+// waves, so that a lane holds few vectors, its chain of arithmetic stays
+// short and a call of few rows still fills CUs.  Rows beyond 16 waves x 16
+// vectors a lane (131072 f16, 65536 f32 columns) are streamed by 16 waves,
+// re-reading the row per pass.  Rows need no alignment: gfx950 takes 16-byte
+// accesses at any element address, and only a row's last partial vector is
+// read and written element by element.
 #include <type_traits>
 
 #include "device_util.h"
@@ -24,49 +27,13 @@ namespace hxm {
 
 enum RowOp { kSoftmax = 0, kRmsNorm = 1, kLayerNorm = 2 };
 
-constexpr int kRowWaves = 4;  // rows (waves) per workgroup
+// Waves of a workgroup whose rows take S waves each.
+constexpr int row_waves(int S) { return S < 4 ? 4 : S; }
 
 template <typename T>
 struct RowVec {
   static constexpr int N = 16 / sizeof(T);  // elements per 16-byte vector
 };
-
-// Loads the 16-byte vector starting at column c0 into f[], padding columns
-// >= cols with `fill`.  ALIGNED means the row base is 16-byte aligned, so a
-// full in-bounds vector is one dwordx4 load.
-template <typename T, bool ALIGNED>
-__device__ __forceinline__ void load_vec(const T* __restrict__ row, int64_t c0,
-                                         int64_t cols, float fill,
-                                         float (&f)[RowVec<T>::N]) {
-  constexpr int N = RowVec<T>::N;
-  if (ALIGNED && c0 + N <= cols) {
-    typedef T vt __attribute__((ext_vector_type(N)));
-    vt v = *reinterpret_cast<const vt*>(row + c0);
-#pragma unroll
-    for (int j = 0; j < N; ++j) f[j] = tof(v[j]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < N; ++j) f[j] = (c0 + j < cols) ? tof(row[c0 + j]) : fill;
-  }
-}
-
-template <typename T, bool ALIGNED>
-__device__ __forceinline__ void store_vec(T* __restrict__ row, int64_t c0,
-                                          int64_t cols,
-                                          const float (&f)[RowVec<T>::N]) {
-  constexpr int N = RowVec<T>::N;
-  if (ALIGNED && c0 + N <= cols) {
-    typedef T vt __attribute__((ext_vector_type(N)));
-    vt v;
-#pragma unroll
-    for (int j = 0; j < N; ++j) v[j] = fromf<T>(f[j]);
-    *reinterpret_cast<vt*>(row + c0) = v;
-  } else {
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-      if (c0 + j < cols) row[c0 + j] = fromf<T>(f[j]);
-  }
-}
 
 // exp(x) for x <= 0 via the hardware exp2 (v_exp_f32): exp(x) = 2^(x*log2 e).
 __device__ __forceinline__ float exp_f32(float x) {
@@ -91,13 +58,10 @@ struct RowArgs {
 template <typename T>
 using RawVec = T __attribute__((ext_vector_type(RowVec<T>::N)));
 
-// Loads the vector at column c0 in storage form, columns >= cols set to
-// `fill`.  ALIGNED (16-byte aligned rows, cols a multiple of N): the vector
-// lies wholly inside the row or wholly past it, and one dwordx4 load reads
-// it.  A lane past the row loads column 0 instead (a valid address) and takes
-// the fill, so no branch splits the wave's loads and all of them are in
-// flight together.
-//
+// The same vector at any element address (a row may start anywhere).
+template <typename T>
+using AnyVec = T __attribute__((ext_vector_type(RowVec<T>::N), aligned(sizeof(T))));
+
 // Row loads are plain (cacheable) and row stores nontemporal.  On a stream
 // that reads and writes HBM at once this pairing ran fastest of the four
 // (64 MiB copy, one box: plain loads + nontemporal stores 20.2 us,
@@ -105,32 +69,50 @@ using RawVec = T __attribute__((ext_vector_type(RowVec<T>::N)));
 // both 24.6); RMSNorm 22.1 -> 20.8 us and softmax 22.9 -> 20.9 us at
 // 8192 x 4096 f16 with nontemporal loads replaced.  A read-only stream is the
 // other way round (the GEMV's weights stay nontemporal).
-template <typename T, bool ALIGNED>
-__device__ __forceinline__ RawVec<T> load_raw(const T* __restrict__ row, int64_t c0,
-                                              int64_t cols, T fill) {
-  constexpr int N = RowVec<T>::N;
-  if constexpr (ALIGNED) {
-    const bool in = c0 < cols;
-    const RawVec<T> v = *reinterpret_cast<const RawVec<T>*>(row + (in ? c0 : 0));
-    return in ? v : RawVec<T>(fill);
-  }
-  RawVec<T> v;
-#pragma unroll
-  for (int j = 0; j < N; ++j) v[j] = (c0 + j < cols) ? row[c0 + j] : fill;
-  return v;
+template <typename T>
+__device__ __forceinline__ RawVec<T> load_any(const T* p) {
+  return *reinterpret_cast<const AnyVec<T>*>(p);
+}
+template <typename T>
+__device__ __forceinline__ void store_any(T* p, RawVec<T> v) {
+  __builtin_nontemporal_store(static_cast<AnyVec<T>>(v), reinterpret_cast<AnyVec<T>*>(p));
 }
 
-template <typename T, bool ALIGNED>
-__device__ __forceinline__ void store_raw(T* __restrict__ row, int64_t c0, int64_t cols,
-                                          RawVec<T> v) {
+// The row's last, partial vector (elements [c0, cols), at least one): element
+// by element, the rest of the vector set to `fill`.
+template <typename T>
+__device__ __forceinline__ RawVec<T> load_tail(const T* __restrict__ row, int64_t c0, int64_t cols,
+                                               T fill) {
   constexpr int N = RowVec<T>::N;
-  if constexpr (ALIGNED) {
-    if (c0 < cols) __builtin_nontemporal_store(v, reinterpret_cast<RawVec<T>*>(row + c0));
-  } else {
+  const int rem = static_cast<int>(cols - c0);
+  RawVec<T> v;
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-      if (c0 + j < cols) row[c0 + j] = v[j];
+  for (int j = 0; j < N; ++j) {
+    const T e = row[c0 + min(j, rem - 1)];
+    v[j] = j < rem ? e : fill;
   }
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ void store_tail(T* __restrict__ row, int64_t c0, int64_t cols,
+                                           RawVec<T> v) {
+#pragma unroll
+  for (int j = 0; j < RowVec<T>::N; ++j)
+    if (c0 + j < cols) row[c0 + j] = v[j];
+}
+
+// The S wave totals of a row combined pairwise (the rounding of S sequential
+// adds of near-equal totals showed in f32 LayerNorm means).
+template <int S, typename Op>
+__device__ __forceinline__ float wave_totals(const float* t, Op op) {
+  float v[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k) v[k] = t[k];
+#pragma unroll
+  for (int w = 1; w < S; w *= 2)
+#pragma unroll
+    for (int k = 0; k + w < S; k += 2 * w) v[k] = op(v[k], v[k + w]);
+  return v[0];
 }
 
 // Makes the compiler treat the row registers as rewritten, so that each pass
@@ -142,36 +124,36 @@ __device__ __forceinline__ void fresh(RawVec<T> (&v)[VPL]) {
   for (int i = 0; i < VPL; ++i) asm volatile("" : "+v"(v[i]));
 }
 
-// Register-resident kernel: each lane holds VPL vectors of the row in the
-// storage type (f16/bf16 rows take half the registers of fp32 copies, so
-// more waves fit per SIMD and more bytes are in flight).  Values are
-// widened to fp32 as each pass reads them.
+// Register-resident kernel: S waves share a row, wave w of the row holding its
+// vectors w, w + S, ... of every 64-lane slot (VPL slots a lane) in the storage
+// type (f16/bf16 rows take half the registers of fp32 copies, so more waves
+// fit per SIMD and more bytes are in flight).  Values are widened to fp32 as
+// each pass reads them.
 //
-// FULL (chosen on the host): the rows are aligned and fill every slot,
-// cols == VPL * 64 * N, so every access is a plain 16-byte vector and no
-// padding logic is compiled.  The kernel that also handles partial rows
-// holds more registers for that logic (LayerNorm f16 at 4096 columns: 107
-// VGPRs, four waves per SIMD, against 62 and eight waves); measured 25.7
-// against 25.2 us (8192 rows, one box).
+// FULL (chosen on the host): the row fills every slot, cols == S * VPL * 64 * N,
+// and no padding logic is compiled.  Measured with one wave per row, LayerNorm
+// f16 at 4096 columns: 107 VGPRs with it, 62 without; 25.7 against 25.2 us.
+// Otherwise the host picks the smallest VPL that holds the row, so that the
+// row's last, partial vector lies in one of the slots [TAIL0, VPL).
 //
-// S > 1 (full rows only): S waves share a row, each holding every S-th
-// vector, and the wave totals meet in LDS behind a barrier.  Each wave's
-// chain of arithmetic after its loads is S times shorter, and that chain is
-// what the last rows of the grid add after the last bytes land.  Every op
-// takes it on full rows of 8 vectors per lane.  Measured (8192 x 4096 f16,
-// one box, two alternating passes each): S = 1 against S = 2, RMSNorm
+// S > 1: the wave totals meet in LDS behind a barrier.  Each wave's chain of
+// arithmetic after its loads is S times shorter, and that chain is what the
+// last rows of the grid add after the last bytes land.  Measured (8192 x 4096
+// f16, one box, two alternating passes each): S = 1 against S = 2, RMSNorm
 // 20.74 -> 20.20 us, LayerNorm 21.77 -> 20.70 us, softmax 20.86 -> 20.88 us;
 // S = 2 against S = 4 (one row per workgroup), softmax 20.87 -> 19.96 us,
-// RMSNorm 19.97 -> 19.84 us, LayerNorm 20.8 -> 20.94 us.  So softmax and
-// RMSNorm take four waves per row and LayerNorm two.  (With nontemporal row
-// loads S = 2 had gained softmax 23.1 -> 22.8 us and cost RMSNorm and
-// LayerNorm 1.5 us each.)
-template <typename T, int OP, int VPL, bool ALIGNED, bool FULL, int S = 1>
-__global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
-  static_assert(!FULL || ALIGNED, "full rows are aligned rows");
-  static_assert(S == 1 || (FULL && kRowWaves % S == 0), "split rows are full rows");
+// RMSNorm 19.97 -> 19.84 us, LayerNorm 20.8 -> 20.94 us (its two dependent
+// reductions each cross the LDS).
+//
+// L < 64: a row is as short as one 16-lane row of the wave and a wave holds
+// 64 / L of them, so short rows do not leave most lanes idle.
+template <typename T, int OP, int VPL, int S, bool FULL, int L = 64>
+__global__ __launch_bounds__(row_waves(S) * 64) void row_kernel(RowArgs a) {
+  static_assert(L == 64 || (L == 16 && S == 1), "short rows: 16 lanes of one wave");
   constexpr int N = RowVec<T>::N;
-  const int lane = threadIdx.x & 63;
+  constexpr int WAVES = row_waves(S);
+  constexpr int TAIL0 = VPL <= 4 ? VPL - 1 : VPL / 2;
+  const int lane = threadIdx.x % L;  // within the row
   const int wv = threadIdx.x >> 6;
   const int half = wv % S;  // this wave's share of the row
   // Softmax takes its row groups XCD-contiguously: workgroups are dispatched
@@ -186,12 +168,13 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
     const int G = gridDim.x, x = blk & 7;
     blk = x * (G >> 3) + min(x, G & 7) + (blk >> 3);
   }
-  const int64_t r = static_cast<int64_t>(blk) * (kRowWaves / S) + wv / S;
-  if constexpr (S == 1) {
+  const int64_t r = static_cast<int64_t>(blk) * (WAVES * (64 / L) / S) +
+                    (L == 64 ? wv / S : static_cast<int>(threadIdx.x) / L);
+  if constexpr (S == 1 && L == 64) {
     if (r >= a.rows) return;  // whole wave leaves; no barriers below
   }
-  // S > 1: a wave past the last row stays for the barriers, reads row 0 and
-  // stores nothing.
+  // Otherwise lanes past the last row stay for the reductions, read row 0 and
+  // store nothing.
   const bool valid = r < a.rows;
   const int64_t rv = valid ? r : 0;
   const T* __restrict__ xr = static_cast<const T*>(a.x) + rv * a.ldx;
@@ -199,53 +182,55 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
   // Row total: the wave's, then (S > 1) the S waves' in a fixed order, so
   // every wave of the row holds the same value.  Each slot serves one
   // reduction of the kernel, so no slot is rewritten after the barrier.
-  __shared__ float red[2][kRowWaves];
+  __shared__ float red[2][WAVES];
   auto row_reduce = [&](float x, auto op, int slot) {
+    if constexpr (L == 16) return row16_reduce(x, op);
     x = wave_reduce(x, op);
     if constexpr (S > 1) {
       if (lane == 0) red[slot][wv] = x;
       __syncthreads();
-      const int base = (wv / S) * S;
-      x = red[slot][base];
-#pragma unroll
-      for (int k = 1; k < S; ++k) x = op(x, red[slot][base + k]);
+      x = wave_totals<S>(red[slot] + (wv / S) * S, op);
     }
     return x;
   };
   const int64_t cols = a.cols;
   const T* __restrict__ g = static_cast<const T*>(a.gamma);
   const T* __restrict__ b = static_cast<const T*>(a.beta);
-  auto col0 = [&](int i) { return ((static_cast<int64_t>(i) * S + half) * 64 + lane) * N; };
+  auto col0 = [&](int i) { return ((static_cast<int64_t>(i) * S + half) * L + lane) * N; };
+  // Slot i holds row elements only (uniform; every slot before TAIL0 does).
+  auto whole = [&](int i) { return FULL || i < TAIL0 || (i + 1) * (S * L * N) <= cols; };
+  // Vector i of a row or of gamma / beta.  A lane past the row (or on its
+  // partial vector) loads column 0 instead, a valid address, and takes the
+  // fill, so that no branch splits the wave's loads and all of them are in
+  // flight together.
+  auto load_at = [&](const T* __restrict__ p, int i, T fill) -> RawVec<T> {
+    if constexpr (FULL) return load_any(p + col0(i));
+    if (i < TAIL0) return load_any(p + col0(i));
+    const int64_t c = col0(i);
+    RawVec<T> v = RawVec<T>(fill);
+    if (cols >= N) {  // uniform
+      const bool in = c + N <= cols;
+      const RawVec<T> t = load_any(p + (in ? c : 0));
+      v = in ? t : v;
+    }
+    if (c < cols && c + N > cols) v = load_tail(p, c, cols, fill);
+    return v;
+  };
+  auto store_at = [&](int i, RawVec<T> v) {
+    if (!valid) return;
+    const int64_t c = col0(i);
+    if (FULL || i < TAIL0 || c + N <= cols) store_any(yr + c, v);
+    else if (c < cols) store_tail(yr, c, cols, v);
+  };
 
   const T fill = static_cast<T>(OP == kSoftmax ? -__builtin_huge_valf() : 0.0f);
-  // A row that fills every slot takes plain loads: with a fill select the
-  // compiler puts each load in its own branch and waits for it before
-  // issuing the next, so one load per wave would be in flight.
-  constexpr bool full = FULL;
-  auto plain = [&](const T* p, int i) {
-    return *reinterpret_cast<const RawVec<T>*>(p + col0(i));
-  };
   RawVec<T> v[VPL];
-  if constexpr (full) {
 #pragma unroll
-    for (int i = 0; i < VPL; ++i)
-      v[i] = *reinterpret_cast<const RawVec<T>*>(xr + col0(i));
-  } else {
-#pragma unroll
-    for (int i = 0; i < VPL; ++i) v[i] = load_raw<T, ALIGNED>(xr, col0(i), cols, fill);
-  }
+  for (int i = 0; i < VPL; ++i) v[i] = load_at(xr, i, fill);
   // gamma / beta vector i, read in the output pass (cache hits: every row
   // shares them), so no registers hold them while the row is in flight.
-  auto gamma_at = [&](int i) {
-    if (!g) return RawVec<T>(T(1));
-    if constexpr (full) return plain(g, i);
-    return load_raw<T, ALIGNED>(g, col0(i), cols, T(0));
-  };
-  auto beta_at = [&](int i) {
-    if (!b) return RawVec<T>(T(0));
-    if constexpr (full) return plain(b, i);
-    return load_raw<T, ALIGNED>(b, col0(i), cols, T(0));
-  };
+  auto gamma_at = [&](int i) { return g ? load_at(g, i, T(0)) : RawVec<T>(T(1)); };
+  auto beta_at = [&](int i) { return b ? load_at(b, i, T(0)) : RawVec<T>(T(0)); };
 
   if constexpr (OP == kSoftmax) {
     // The row maximum is exact in the storage type, so f16 rows take it with
@@ -313,7 +298,7 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
         asm volatile("" : "+v"(p));
         o[j] = fromf<T>(p);
       }
-      if (valid) store_raw<T, ALIGNED>(yr, col0(i), cols, o);
+      store_at(i, o);
     }
   } else if constexpr (OP == kRmsNorm) {
     // Every pass is written as fmas whose f16 operands gfx950 takes straight
@@ -342,7 +327,7 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
 #pragma unroll
       for (int j = 0; j < N; ++j)
         o[j] = fromf<T>(fmaf(fmaf(tof(v[i][j]), rstd, nzero), tof(gi[j]), nzero));
-      if (valid) store_raw<T, ALIGNED>(yr, col0(i), cols, o);
+      store_at(i, o);
     }
   } else {  // kLayerNorm
     // The row is widened into mixed-precision fmas as in RMSNorm: the sum as
@@ -368,31 +353,25 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
     const float mean = row_reduce(s, OpSum(), 0) / static_cast<float>(cols);
     const float nmean = -mean;
     fresh(v);
-    // Padding slots (columns >= cols, loaded as 0) must not add mean^2: a
-    // row that fills every slot (a uniform branch) skips the per-element
-    // test.  Measured (8192 x 4096 f16, one box): this form 27.2 us, a
-    // per-vector test on partial sums 27.9 us (it frees registers, 65
-    // instead of 108 VGPRs, but the extra waves do not help), per-element
-    // test with a branch around every load 28.5-29.1 us.
+    // Padding slots (columns >= cols, loaded as 0) must not add mean^2: only
+    // slots that are not whole take the per-element test.
     float q = 0.0f;
-    if (full || cols == static_cast<int64_t>(VPL) * 64 * N) {
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) {
+    for (int i = 0; i < VPL; ++i) {
+      if (whole(i)) {
 #pragma unroll
         for (int j = 0; j < N; ++j) {
           const float d = fmaf(tof(v[i][j]), one, nmean);
           q = fmaf(d, d, q);
         }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < VPL; ++i)
+      } else {
 #pragma unroll
         for (int j = 0; j < N; ++j) {
           const float d = (col0(i) + j < cols) ? fmaf(tof(v[i][j]), one, nmean) : 0.0f;
           q = fmaf(d, d, q);
         }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     const float var = row_reduce(q, OpSum(), 1) / static_cast<float>(cols);
     fresh(v);
@@ -410,176 +389,223 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
         const float d = fmaf(tof(v[i][j]), one, nmean);
         o[j] = fromf<T>(fmaf(d * rstd, tof(gi[j]), tof(bi[j])));
       }
-      if (valid) store_raw<T, ALIGNED>(yr, col0(i), cols, o);
+      store_at(i, o);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
 
-// Streaming kernel for rows longer than the register budget: the row is
-// re-read per pass (softmax 3: max, sum of rounded numerators, output;
-// RMSNorm 2, LayerNorm 3).
-template <typename T, int OP, bool ALIGNED>
-__global__ __launch_bounds__(256) void row_kernel_stream(RowArgs a) {
+// Streaming kernel for rows longer than the register budget: S waves share a
+// row and re-read it per pass (softmax 3: max, sum of rounded numerators,
+// output; RMSNorm 2, LayerNorm 3).
+//
+// f32 LayerNorm above 4096 columns keeps one wave per row (registers to 8192
+// columns, then this kernel with S = 1): the mean of a long row is the
+// difference of near-equal sums, and its fp32 rounding in another order (a few
+// 1e-6 of a mean near zero at 1e5 columns) would show in the mean and rstd
+// that callers keep for the backward pass.  Eight loads in flight: 175 x 50688
+// 229 -> 88 us, 4096 x 8192 (registers) 75.7 -> 47.3.
+template <typename T, int OP, int S>
+__global__ __launch_bounds__(S * 64) void row_kernel_stream(RowArgs a) {
   constexpr int N = RowVec<T>::N;
-  const int lane = threadIdx.x & 63;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * kRowWaves + (threadIdx.x >> 6);
-  if (r >= a.rows) return;
+  const int64_t r = blockIdx.x;
   const T* __restrict__ xr = static_cast<const T*>(a.x) + r * a.ldx;
   T* __restrict__ yr = static_cast<T*>(a.y) + r * a.ldy;
   const int64_t cols = a.cols;
-  const int64_t step = 64 * N;
   const T* __restrict__ g = static_cast<const T*>(a.gamma);
   const T* __restrict__ b = static_cast<const T*>(a.beta);
+  __shared__ float red[2][S];
+  auto row_reduce = [&](float x, auto op, int slot) {
+    x = wave_reduce(x, op);
+    if constexpr (S == 1) return x;
+    if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = x;
+    __syncthreads();
+    return wave_totals<S>(red[slot], op);
+  };
+  // f(c0, vector, elements of it inside the row) over this thread's vectors.
+  auto each = [&](T fill, auto f) {
+    const int64_t nfull = cols / N;
+    int64_t i = threadIdx.x;
+    for (; i + 7 * S * 64 < nfull; i += 8 * S * 64) {  // eight loads in flight
+      RawVec<T> v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = load_any(xr + (i + u * S * 64) * N);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) f((i + u * S * 64) * N, v[u], N);
+    }
+    for (; i < nfull; i += S * 64) f(i * N, load_any(xr + i * N), N);
+    const int rem = static_cast<int>(cols - nfull * N);
+    if (rem && static_cast<int64_t>(threadIdx.x) == nfull % (S * 64))
+      f(nfull * N, load_tail(xr, nfull * N, cols, fill), rem);
+  };
+  auto store = [&](int64_t c0, RawVec<T> v, int n) {
+    if (n == N) store_any(yr + c0, v);
+    else store_tail(yr, c0, cols, v);
+  };
+  auto param = [&](const T* p, int64_t c0, int n, T none) -> RawVec<T> {
+    if (!p) return RawVec<T>(none);
+    return n == N ? load_any(p + c0) : load_tail(p, c0, cols, none);
+  };
 
-  float scale = 1.0f, shift = 0.0f;  // y = (x - shift) * scale [* g + b]
-  float m = 0.0f;
   if constexpr (OP == kSoftmax) {
     // The row max, then the fp32 sum of the numerators rounded to the
     // storage type (the reference's arithmetic, as in row_kernel): an online
     // max/sum would rescale sums of unrounded numerators instead.
-    float lm = -__builtin_huge_valf();
-    for (int64_t c0 = lane * N; c0 < cols; c0 += step) {
-      float f[N];
-      load_vec<T, ALIGNED>(xr, c0, cols, -__builtin_huge_valf(), f);
+    float m = -__builtin_huge_valf();
+    each(static_cast<T>(-__builtin_huge_valf()), [&](int64_t, RawVec<T> v, int) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) lm = fmaxf(lm, f[j]);
-    }
-    m = wave_reduce(lm, OpMax());
-    float ls = 0.0f;
-    for (int64_t c0 = lane * N; c0 < cols; c0 += step) {
-      float f[N];
-      load_vec<T, ALIGNED>(xr, c0, cols, -__builtin_huge_valf(), f);
+      for (int j = 0; j < N; ++j) m = fmaxf(m, tof(v[j]));
+    });
+    m = row_reduce(m, OpMax(), 0);
+    float s = 0.0f;
+    each(static_cast<T>(-__builtin_huge_valf()), [&](int64_t, RawVec<T> v, int n) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) ls += tof(fromf<T>(exp_f32(f[j] - m)));
-    }
-    const float s = wave_reduce(ls, OpSum());
-    scale = 1.0f / s;
+      for (int j = 0; j < N; ++j) s += j < n ? tof(fromf<T>(exp_f32(tof(v[j]) - m))) : 0.0f;
+    });
+    s = row_reduce(s, OpSum(), 1);
+    const float scale = 1.0f / s;
+    each(T(0), [&](int64_t c0, RawVec<T> v, int n) {
+      RawVec<T> o;
+#pragma unroll
+      for (int j = 0; j < N; ++j) o[j] = fromf<T>(tof(fromf<T>(exp_f32(tof(v[j]) - m))) * scale);
+      store(c0, o, n);
+    });
   } else if constexpr (OP == kRmsNorm) {
     float ss = 0.0f;
-    for (int64_t c0 = lane * N; c0 < cols; c0 += step) {
-      float f[N];
-      load_vec<T, ALIGNED>(xr, c0, cols, 0.0f, f);
+    each(T(0), [&](int64_t, RawVec<T> v, int) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) ss += f[j] * f[j];
-    }
-    ss = wave_reduce(ss, OpSum());
-    scale = 1.0f / sqrtf(ss / static_cast<float>(cols) + a.eps);
+      for (int j = 0; j < N; ++j) ss += tof(v[j]) * tof(v[j]);
+    });
+    ss = row_reduce(ss, OpSum(), 0);
+    const float scale = 1.0f / sqrtf(ss / static_cast<float>(cols) + a.eps);
+    each(T(0), [&](int64_t c0, RawVec<T> v, int n) {
+      const RawVec<T> gv = param(g, c0, n, T(1));
+      RawVec<T> o;
+#pragma unroll
+      for (int j = 0; j < N; ++j) o[j] = fromf<T>((tof(v[j]) * scale) * tof(gv[j]));
+      store(c0, o, n);
+    });
   } else {
     float s = 0.0f;
-    for (int64_t c0 = lane * N; c0 < cols; c0 += step) {
-      float f[N];
-      load_vec<T, ALIGNED>(xr, c0, cols, 0.0f, f);
+    each(T(0), [&](int64_t, RawVec<T> v, int) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) s += f[j];
-    }
-    const float mean = wave_reduce(s, OpSum()) / static_cast<float>(cols);
+      for (int j = 0; j < N; ++j) s += tof(v[j]);
+    });
+    const float mean = row_reduce(s, OpSum(), 0) / static_cast<float>(cols);
     float q = 0.0f;
-    for (int64_t c0 = lane * N; c0 < cols; c0 += step) {
-      float f[N];
-      load_vec<T, ALIGNED>(xr, c0, cols, 0.0f, f);
+    each(T(0), [&](int64_t, RawVec<T> v, int n) {
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-        const float d = (c0 + j < cols) ? f[j] - mean : 0.0f;
+        const float d = j < n ? tof(v[j]) - mean : 0.0f;
         q += d * d;
       }
-    }
-    const float var = wave_reduce(q, OpSum()) / static_cast<float>(cols);
-    shift = mean;
-    scale = 1.0f / sqrtf(var + a.eps);
-    if (lane == 0) {
+    });
+    const float var = row_reduce(q, OpSum(), 1) / static_cast<float>(cols);
+    const float rstd = 1.0f / sqrtf(var + a.eps);
+    if (threadIdx.x == 0) {
       if (a.mean_out) a.mean_out[r] = mean;
-      if (a.rstd_out) a.rstd_out[r] = scale;
+      if (a.rstd_out) a.rstd_out[r] = rstd;
     }
-  }
-
-  for (int64_t c0 = lane * N; c0 < cols; c0 += step) {
-    float f[N];
-    load_vec<T, ALIGNED>(xr, c0, cols, 0.0f, f);
-    if constexpr (OP == kSoftmax) {
-#pragma unroll
-      for (int j = 0; j < N; ++j) f[j] = tof(fromf<T>(exp_f32(f[j] - m))) * scale;
-    } else if constexpr (OP == kRmsNorm) {
-      float gv[N];
-      if (g) load_vec<T, ALIGNED>(g, c0, cols, 0.0f, gv);
-#pragma unroll
-      for (int j = 0; j < N; ++j) f[j] = (f[j] * scale) * (g ? gv[j] : 1.0f);
-    } else {
-      float gv[N], bv[N];
-      if (g) load_vec<T, ALIGNED>(g, c0, cols, 0.0f, gv);
-      if (b) load_vec<T, ALIGNED>(b, c0, cols, 0.0f, bv);
+    each(T(0), [&](int64_t c0, RawVec<T> v, int n) {
+      const RawVec<T> gv = param(g, c0, n, T(1)), bv = param(b, c0, n, T(0));
+      RawVec<T> o;
 #pragma unroll
       for (int j = 0; j < N; ++j)
-        f[j] = (f[j] - shift) * scale * (g ? gv[j] : 1.0f) + (b ? bv[j] : 0.0f);
-    }
-    store_vec<T, ALIGNED>(yr, c0, cols, f);
+        o[j] = fromf<T>((tof(v[j]) - mean) * rstd * tof(gv[j]) + tof(bv[j]));
+      store(c0, o, n);
+    });
   }
 }
 
 namespace {
 
-template <typename T, int OP, bool ALIGNED>
+// Waves per row (S) and 16-byte vectors per lane (VPL) by the row's vectors:
+// the fewest slots that hold the row, three or four a lane before the next S
+// (one wave up to 256 vectors, where the whole chip's rows are short enough:
+// 8192 x 2048 f16 8.6 us with one wave a row, 10.1 with two).  Rows below 64
+// vectors share a wave four at a time once there are enough of them to fill
+// the chip that way (20000 x 300 f16 softmax 8.3 -> 5.8 us, 60000 x 64 14.9 ->
+// 5.0; 100 x 300 2.5 -> 2.7).  Before, every row had one wave, unaligned rows
+// were read element by element and rows above 1024 vectors re-read per pass
+// (softmax / RMSNorm / LayerNorm, one box, HIP graph): f16 2047 x 5003 30.9 /
+// 38.8 / 48.7 -> 8.3 / 8.4 / 9.7 us, 85 x 16857 85.0 / 77.6 / 122.2 -> 5.8 /
+// 5.0 / 6.5, 2048 x 16384 50.2 / 42.1 / 66.0 -> 22.2 / 20.1 / 20.7, f32 4096 x
+// 8192 75.9 / 57.6 / 75.3 -> 39.4 / 38.9 / 47.3, 175 x 50688 207.7 / 153.4 /
+// 229.3 -> 14.4 / 13.4 / 88.
+constexpr int64_t kShortRowsMin = 2048;
+template <typename T, int OP>
 hxm_status launch_rows_t(const RowArgs& a, hipStream_t stream) {
   constexpr int N = RowVec<T>::N;
-  const int64_t vpl = (a.cols + 64 * N - 1) / (64 * N);
-  // Full rows of 8 vectors per lane: SPLIT waves per row, four for softmax
-  // and RMSNorm, two for LayerNorm (its two dependent reductions cross the
-  // LDS twice).
-  constexpr int SPLIT = OP == kLayerNorm ? 2 : 4;
-  const bool split = ALIGNED && a.cols == 8 * 64 * N;
-  const int64_t rows_per_group = split ? kRowWaves / SPLIT : kRowWaves;
-  const int64_t groups = (a.rows + rows_per_group - 1) / rows_per_group;
-  hxm_status st = check_grid("row kernel", groups, 64 * kRowWaves);
-  if (st != HXM_OK) return st;
-  const dim3 grid(static_cast<unsigned>(groups));
-  const dim3 block(64 * kRowWaves);
-  // FULL kernels for aligned rows that fill the VPL slots exactly.
-  auto run = [&](auto VPLC) {
-    constexpr int V = decltype(VPLC)::value;
-    if constexpr (ALIGNED && V == 8) {
-      if (split) {
-        row_kernel<T, OP, V / SPLIT, true, true, SPLIT><<<grid, block, 0, stream>>>(a);
-        return;
-      }
+  const int64_t nv = (a.cols + N - 1) / N;
+  hxm_status st = HXM_OK;
+  // Rows one call may hold: four to a 256-thread workgroup (the full rows of
+  // 512 vectors: their own one or two) within the launch limit.  Wider
+  // workgroups launch in as many pieces as that takes.
+  auto launch = [&](auto kernel, int threads, int per_group, int per_group_limit) {
+    if ((st = check_grid("row kernel", (a.rows + per_group_limit - 1) / per_group_limit, 256)) !=
+        HXM_OK)
+      return;
+    const int64_t piece = (0xffffffffLL / threads) * per_group;
+    for (int64_t r = 0; r < a.rows; r += piece) {
+      RowArgs p = a;
+      p.x = static_cast<const T*>(a.x) + r * a.ldx;
+      p.y = static_cast<T*>(a.y) + r * a.ldy;
+      if (a.mean_out) p.mean_out = a.mean_out + r;
+      if (a.rstd_out) p.rstd_out = a.rstd_out + r;
+      p.rows = a.rows - r < piece ? a.rows - r : piece;
+      const int64_t groups = (p.rows + per_group - 1) / per_group;
+      kernel<<<dim3(static_cast<unsigned>(groups)), dim3(threads), 0, stream>>>(p);
     }
-    if (ALIGNED && a.cols == static_cast<int64_t>(V) * 64 * N)
-      row_kernel<T, OP, V, ALIGNED, ALIGNED><<<grid, block, 0, stream>>>(a);
-    else
-      row_kernel<T, OP, V, ALIGNED, false><<<grid, block, 0, stream>>>(a);
   };
-  if (vpl <= 1)
-    run(std::integral_constant<int, 1>{});
-  else if (vpl <= 2)
-    run(std::integral_constant<int, 2>{});
-  else if (vpl <= 4)
-    run(std::integral_constant<int, 4>{});
-  else if (vpl <= 8)
-    run(std::integral_constant<int, 8>{});
-  else if (vpl <= 16)
-    run(std::integral_constant<int, 16>{});
-  else
-    row_kernel_stream<T, OP, ALIGNED><<<grid, block, 0, stream>>>(a);
+  auto run = [&](auto VC, auto SC, auto LC) {
+    constexpr int V = decltype(VC)::value, S = decltype(SC)::value, L = decltype(LC)::value;
+    constexpr int per_group = row_waves(S) * (64 / L) / S;
+    if (a.cols == static_cast<int64_t>(V) * S * L * N)
+      launch(row_kernel<T, OP, V, S, true, L>, 64 * row_waves(S), per_group,
+             nv == 512 ? per_group : 4);
+    else
+      launch(row_kernel<T, OP, V, S, false, L>, 64 * row_waves(S), per_group, 4);
+  };
+#define HXM_ROWS_L(V, S, L)                                                        \
+  run(std::integral_constant<int, V>{}, std::integral_constant<int, S>{}, \
+      std::integral_constant<int, L>{})
+#define HXM_ROWS(V, S) HXM_ROWS_L(V, S, 64)
+  const bool shared = a.rows >= kShortRowsMin;
+  if (shared && nv <= 16) HXM_ROWS_L(1, 1, 16);
+  else if (shared && nv <= 32) HXM_ROWS_L(2, 1, 16);
+  else if (shared && nv <= 48) HXM_ROWS_L(3, 1, 16);
+  else if (shared && nv < 64) HXM_ROWS_L(4, 1, 16);
+  else if (nv <= 64) HXM_ROWS(1, 1);
+  else if (nv <= 128) HXM_ROWS(2, 1);
+  else if (nv <= 192) HXM_ROWS(3, 1);
+  else if (nv <= 256) HXM_ROWS(4, 1);
+  else if (OP == kLayerNorm && nv <= 384) HXM_ROWS(3, 2);
+  else if (OP == kLayerNorm && nv <= 512) HXM_ROWS(4, 2);
+  else if (nv <= 512) HXM_ROWS(2, 4);
+  else if (nv <= 768) HXM_ROWS(3, 4);
+  else if (nv <= 1024) HXM_ROWS(4, 4);
+  else if (OP == kLayerNorm && sizeof(T) == 4 && nv <= 1536) HXM_ROWS(24, 1);
+  else if (OP == kLayerNorm && sizeof(T) == 4 && nv <= 2048) HXM_ROWS(32, 1);
+  else if (OP == kLayerNorm && sizeof(T) == 4) launch(row_kernel_stream<T, OP, 1>, 64, 1, 4);
+  else if (nv <= 1536) HXM_ROWS(3, 8);
+  else if (nv <= 2048) HXM_ROWS(4, 8);
+  else if (nv <= 3072) HXM_ROWS(3, 16);
+  else if (nv <= 4096) HXM_ROWS(4, 16);
+  else if (nv <= 8192) HXM_ROWS(8, 16);
+  else if (nv <= 16384) HXM_ROWS(16, 16);
+  else launch(row_kernel_stream<T, OP, 16>, 1024, 1, 4);
+#undef HXM_ROWS
+#undef HXM_ROWS_L
+  if (st != HXM_OK) return st;
   return check_launch("row kernel");
 }
 
 template <int OP>
 hxm_status launch_rows(const RowArgs& a, int32_t dtype, hipStream_t stream) {
-  const int64_t eb = dtype_bytes(dtype);
-  // ALIGNED kernels: 16-byte aligned rows whose length is a whole number of
-  // 16-byte vectors.
-  bool al = aligned16(a.x) && aligned16(a.y) && (a.ldx * eb) % 16 == 0 &&
-            (a.ldy * eb) % 16 == 0 && (!a.gamma || aligned16(a.gamma)) &&
-            (!a.beta || aligned16(a.beta)) && (a.cols * eb) % 16 == 0;
   switch (dtype) {
-    case HXM_F16:
-      return al ? launch_rows_t<_Float16, OP, true>(a, stream)
-                : launch_rows_t<_Float16, OP, false>(a, stream);
-    case HXM_BF16:
-      return al ? launch_rows_t<__bf16, OP, true>(a, stream)
-                : launch_rows_t<__bf16, OP, false>(a, stream);
-    default:
-      return al ? launch_rows_t<float, OP, true>(a, stream)
-                : launch_rows_t<float, OP, false>(a, stream);
+    case HXM_F16: return launch_rows_t<_Float16, OP>(a, stream);
+    case HXM_BF16: return launch_rows_t<__bf16, OP>(a, stream);
+    default: return launch_rows_t<float, OP>(a, stream);
   }
 }
 
