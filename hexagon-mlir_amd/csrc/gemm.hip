@@ -2,7 +2,7 @@
 // (tuned winner, else a default per shape), argument validation, the [K,N]
 // weight pack and the extern "C" entry points.  The kernels themselves are
 // in gemm_kernel.h, instantiated by gemm_i8.hip, gemm_f16.hip and
-// gemm_w8.hip.
+// gemm_w8.hip; the operand packs in pack.hip.
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -11,81 +11,6 @@
 #include "gemm_kernel.h"
 
 namespace hxm {
-
-// Transpose [K,N] -> [N,K] (the resident weight image).  32x32 element tiles
-// through LDS.
-template <typename E>
-__global__ __launch_bounds__(256) void transpose_kernel(const E* __restrict__ src,
-                                                        int64_t lds_, E* __restrict__ dst,
-                                                        int64_t ldd, int64_t K,
-                                                        int64_t N) {
-  __shared__ E tile[32][33];
-  const int64_t k0 = static_cast<int64_t>(blockIdx.y) * 32;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-#pragma unroll
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t k = k0 + r, n = n0 + tx;
-    if (k < K && n < N) tile[r][tx] = src[k * lds_ + n];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t n = n0 + r, k = k0 + tx;
-    if (n < N && k < K) dst[n * ldd + k] = tile[tx][r];
-  }
-}
-
-// f32 operands of a matmul enter the fp16 MFMA through these packs (the
-// reference's hmx_pack_act_f32 / hmx_pack_weight_f32, HMXAPI.h:107-137,
-// which quantise in the pack; its host prepack spells the conversion as
-// x + 0.0f -- -0 becomes +0 -- then IEEE round to nearest even,
-// hmx_weight_prepack.py:196-207).  The images are fp16 with rows of kp
-// elements, kp = K rounded up to 8 (16-byte rows for the LDS-DMA); the
-// padding columns hold +0, which adds nothing to any sum.
-__device__ __forceinline__ _Float16 f32_operand_to_f16(float x) {
-  return static_cast<_Float16>(x + 0.0f);
-}
-
-// Row-major [rows, cols] f32 (row stride ld) -> [rows, kp] f16.  Each unit
-// is 8 output elements (one 16-byte store).
-__global__ __launch_bounds__(256) void pack_f32_rows_kernel(const float* __restrict__ src,
-                                                            int64_t ld, _Float16* __restrict__ dst,
-                                                            int64_t rows, int64_t cols,
-                                                            int64_t kp) {
-  const int64_t units = rows * (kp / 8);
-  for (int64_t u = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; u < units;
-       u += static_cast<int64_t>(gridDim.x) * 256) {
-    const int64_t r = u / (kp / 8), c0 = (u % (kp / 8)) * 8;
-    v8f16 h;
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      h[e] = c0 + e < cols ? f32_operand_to_f16(src[r * ld + c0 + e]) : static_cast<_Float16>(0.0f);
-    *reinterpret_cast<v8f16*>(dst + r * kp + c0) = h;
-  }
-}
-
-// [K, N] f32 (row stride ld) -> the [N, kp] f16 image, 32 x 32 tiles through
-// LDS; image columns k in [K, kp) are +0.
-__global__ __launch_bounds__(256) void pack_f32_kn_kernel(const float* __restrict__ src,
-                                                          int64_t ld, _Float16* __restrict__ dst,
-                                                          int64_t K, int64_t N, int64_t kp) {
-  __shared__ float tile[32][33];
-  const int64_t k0 = static_cast<int64_t>(blockIdx.y) * 32;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-#pragma unroll
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t k = k0 + r, n = n0 + tx;
-    tile[r][tx] = k < K && n < N ? src[k * ld + n] : 0.0f;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t n = n0 + r, k = k0 + tx;
-    if (n < N && k < kp) dst[n * kp + k] = f32_operand_to_f16(tile[tx][r]);
-  }
-}
 
 // ------------------------------------------------------------------------
 // Host side: the compiled-config table and dispatch.
@@ -290,14 +215,7 @@ hxm_status resolve_b(const void* B, int64_t ldb, int32_t b_layout, int64_t K,
   const int64_t ldo = kn_image_ld(K, eb);
   if ((st = stream_workspace(stream, static_cast<size_t>(N * ldo * eb), &ws)) != HXM_OK)
     return st;
-  const dim3 grid(static_cast<unsigned>((N + 31) / 32), static_cast<unsigned>((K + 31) / 32));
-  if (eb == 1)
-    transpose_kernel<uint8_t><<<grid, 256, 0, stream>>>(
-        static_cast<const uint8_t*>(B), ldb, static_cast<uint8_t*>(ws), ldo, K, N);
-  else
-    transpose_kernel<uint16_t><<<grid, 256, 0, stream>>>(
-        static_cast<const uint16_t*>(B), ldb, static_cast<uint16_t*>(ws), ldo, K, N);
-  if ((st = check_launch("weight pack")) != HXM_OK) return st;
+  if ((st = pack_kn_image(B, ldb, ws, ldo, K, N, eb, stream, "weight pack")) != HXM_OK) return st;
   *b_out = static_cast<const uint8_t*>(ws);
   *ldb_bytes_out = ldo * eb;
   return HXM_OK;
@@ -946,20 +864,9 @@ static hxm_status matmul_f32(const float* A, int64_t lda, const float* B, int64_
     if ((st = stream_workspace(stream, static_cast<size_t>(img_bytes), &ws)) != HXM_OK) return st;
     ai = static_cast<_Float16*>(ws);
     bi = reinterpret_cast<_Float16*>(static_cast<char*>(ws) + a_bytes);
-    auto blocks = [](int64_t units) {
-      return static_cast<unsigned>(std::min<int64_t>((units + 255) / 256, 65536));
-    };
-    pack_f32_rows_kernel<<<blocks(M * (kp / 8)), 256, 0, stream>>>(A, lda, ai, M, K, kp);
-    if ((st = check_launch("f32 operand pack")) != HXM_OK) return st;
-    if (b_layout == HXM_B_NK) {
-      pack_f32_rows_kernel<<<blocks(N * (kp / 8)), 256, 0, stream>>>(B, ldb, bi, N, K, kp);
-    } else {
-      if ((st = check_grid("f32 weight pack", (N + 31) / 32, 256, (kp + 31) / 32)) != HXM_OK)
-        return st;
-      const dim3 grid(static_cast<unsigned>((N + 31) / 32), static_cast<unsigned>((kp + 31) / 32));
-      pack_f32_kn_kernel<<<grid, 256, 0, stream>>>(B, ldb, bi, K, N, kp);
-    }
-    if ((st = check_launch("f32 operand pack")) != HXM_OK) return st;
+    if ((st = pack_f32_operands(A, lda, ai, M, B, ldb, bi, N, K, kp, b_layout == HXM_B_KN,
+                                stream)) != HXM_OK)
+      return st;
   }
   return run_gemm_with(HXM_F32, HXM_F16, kEpiFloat, ai, kp, bi, kp, HXM_B_NK, C, ldc, M, N, kp,
                        c_dtype, accumulate, nullptr, nullptr, cfg, stream, nullptr, 0,
@@ -1056,16 +963,7 @@ hxm_status hxm_prepack_weight(const void* B, int64_t ldb, void* out,
   hxm_status st = require_device(nullptr);
   if (st != HXM_OK) return st;
   if (K == 0 || N == 0) return ok();
-  if ((st = check_grid("prepack", (N + 31) / 32, 256, (K + 31) / 32)) != HXM_OK) return st;
-  hipStream_t s = as_stream(stream);
-  const dim3 grid(static_cast<unsigned>((N + 31) / 32), static_cast<unsigned>((K + 31) / 32));
-  if (dtype == HXM_I8)
-    transpose_kernel<uint8_t><<<grid, 256, 0, s>>>(static_cast<const uint8_t*>(B), ldb,
-                                                   static_cast<uint8_t*>(out), ldo, K, N);
-  else
-    transpose_kernel<uint16_t><<<grid, 256, 0, s>>>(static_cast<const uint16_t*>(B), ldb,
-                                                    static_cast<uint16_t*>(out), ldo, K, N);
-  return check_launch("prepack");
+  return pack_kn_image(B, ldb, out, ldo, K, N, dtype == HXM_I8 ? 1 : 2, as_stream(stream), "prepack");
 }
 
 hxm_status hxm_gemm_w8a16(const void* x, int64_t ldx, const int8_t* W, int64_t ldw,

@@ -91,6 +91,18 @@ hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const
                              int64_t K, int32_t out_dtype, int32_t accumulate,
                              hipStream_t stream);
 
+// Operand packs (pack.hip).  [K, N] (elements of eb = 1 or 2 bytes, row stride
+// ldb) -> the [N, K] image of row stride ldo; the same from f32 to fp16; and the
+// fp16 images of both operands of an f32 matmul ([M, kp] and [N, kp], kp = K
+// rounded up to 8, zero past K) in one launch.
+hxm_status pack_kn_image(const void* B, int64_t ldb, void* out, int64_t ldo, int64_t K, int64_t N,
+                         int64_t eb, hipStream_t stream, const char* what);
+hxm_status pack_kn_f32_image(const float* B, int64_t ldb, _Float16* out, int64_t ldo, int64_t K,
+                             int64_t N, hipStream_t stream);
+hxm_status pack_f32_operands(const float* A, int64_t lda, _Float16* ai, int64_t M, const float* B,
+                             int64_t ldb, _Float16* bi, int64_t N, int64_t K, int64_t kp, bool kn,
+                             hipStream_t stream);
+
 // The skinny W8A16 matmul (gemm_skinny.hip): the default of the W8A16 GEMMs at
 // 1 to kSkinnyRowsMax rows; a caller names it with skinny_config().
 constexpr int64_t kSkinnyRowsMax = 64;

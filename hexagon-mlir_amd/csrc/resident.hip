@@ -62,27 +62,6 @@ __global__ __launch_bounds__(256) void hash_kernel(const uint8_t* __restrict__ s
 
 __global__ void zero2_kernel(unsigned long long* p) { p[threadIdx.x] = 0; }
 
-// [K, N] fp32 (row stride ld) -> [N, K] fp16 image: -0 canonicalised to +0
-// (x + 0.0f), then IEEE round to nearest even.  32 x 32 tiles through LDS.
-__global__ __launch_bounds__(256) void f32_to_f16_image_kernel(const float* __restrict__ src,
-                                                               int64_t ld,
-                                                               _Float16* __restrict__ dst,
-                                                               int64_t K, int64_t N) {
-  __shared__ float tile[32][33];
-  const int64_t k0 = static_cast<int64_t>(blockIdx.y) * 32;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t k = k0 + r, n = n0 + tx;
-    if (k < K && n < N) tile[r][tx] = src[k * ld + n];
-  }
-  __syncthreads();
-  for (int r = ty; r < 32; r += 8) {
-    const int64_t n = n0 + r, k = k0 + tx;
-    if (n < N && k < K) dst[n * K + k] = static_cast<_Float16>(tile[tx][r] + 0.0f);
-  }
-}
-
 struct Image {
   void* ptr = nullptr;
   int32_t dtype = 0;
@@ -195,15 +174,8 @@ hxm_status hxm_resident_weight(const void* src, int64_t ld, int64_t rows, int64_
       st = hxm_prepack_w8a16(static_cast<const int8_t*>(src), ld, rows, cols,
                              static_cast<int8_t*>(img.ptr), bytes, stream);
     } else if (src_dtype == HXM_F32) {
-      if ((st = check_grid("f32 weight image", (cols + 31) / 32, 256, (rows + 31) / 32)) !=
-          HXM_OK)
-        return st;
-      const dim3 grid(static_cast<unsigned>((cols + 31) / 32),
-                      static_cast<unsigned>((rows + 31) / 32));
-      f32_to_f16_image_kernel<<<grid, 256, 0, s>>>(static_cast<const float*>(src), ld,
-                                                   static_cast<_Float16*>(img.ptr), rows,
-                                                   cols);
-      st = check_launch("f32 weight image");
+      st = pack_kn_f32_image(static_cast<const float*>(src), ld, static_cast<_Float16*>(img.ptr),
+                             rows, rows, cols, s);
     } else {
       st = hxm_prepack_weight(src, ld, img.ptr, rows, rows, cols, src_dtype, stream);
     }
