@@ -4,6 +4,7 @@
 // in gemm_kernel.h, instantiated by gemm_i8.hip, gemm_f16.hip and
 // gemm_w8.hip; the operand packs in pack.hip.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -70,29 +71,51 @@ const KernelEntry* find_kernel(const hxm_gemm_config& c, int32_t dt) {
   return nullptr;
 }
 
-// Default configuration for a shape (used when no tuned winner is cached):
-// the first entry of this preference list whose tile count still gives every
-// CU a workgroup, else a small tile (below).
-hxm_gemm_config default_config(int64_t M, int64_t N, int32_t dt) {
-  // bm, bn, bk bytes, stages.  The two-stage 256x256 tile with 128-byte K
-  // stages leads for every dtype (measured at 4096^3: f16 110 us against
-  // 112 us for the four-stage 64-byte tile, bf16 98 against 104 us).
-  static const int order_i8[][4] = {{256, 256, 128, 2}, {256, 256, 64, 4}, {128, 128, 128, 2}};
-  static const int order_f16[][4] = {{256, 256, 128, 2}, {256, 256, 64, 4}, {128, 128, 128, 2}};
-  for (auto& o : (dt == HXM_I8 ? order_i8 : order_f16)) {
-    const int64_t tiles = ((M + o[0] - 1) / o[0]) * ((N + o[1] - 1) / o[1]);
-    if (tiles >= 256) {
-      hxm_gemm_config c{o[0], o[1], o[2] / elem_bytes(dt), 0, 0, o[3], 1};
-      if (find_kernel(c, dt)) return kernel_config(static_cast<int>(find_kernel(c, dt) - kKernels), dt);
-    }
+// Default configuration for a shape (used when no tuned winner is cached): the
+// tile with the least modeled time.  A call runs `rounds` of the workgroups
+// that fit the chip at once (occ per CU), each one fixed time (launch,
+// prologue, epilogue) plus its K stages of 128 bytes; a stage costs stage_lo
+// on an otherwise idle chip (latency, issue) and stage_hi on a full one (L2 ->
+// LDS bandwidth, clock).  int8 and f16/bf16 stages of the same bytes take the
+// same time.  Fitted to tuner measurements (us, one box; modeled / measured):
+//   f16 512 x 4096 x 4096: 128x64 26 / 23.8, 64x64 31 / 28.6, 128x128 36 / 26.9
+//     (two-stage 64x64, the default before: 35.3)
+//   bf16 1776 x 1640 x 4448: 128x128 41 / 40.1, 128x64 51 / 56 (before: 52.0)
+//   f16 3000 cube: 256x256 73 / 73.7, 128x128 89 / 93 (before: 109.7)
+//   int8 1000 x 1500 x 4112: 128x64 14 / 17.4, 128x128 20 / 18.9 (before: 22.3)
+//   int8 3000 x 3000 x 3008: 256x256 38 / 40.1, 128x128 49 / 47 (before: 56.2)
+//   f16 1024 x 4096 x 4096: 128x128 40 / 36.5, 256x128 56 / 41.6 (before: 44.8)
+//   f16 128 x 4096 x 4096: 64x64 19 / 16.9, 128x64 20 / 20.1 (before: 31.8)
+// The deeper prefetch of the small tiles is what they gain: with two stages a
+// 64x64 tile has 32 KiB a CU in flight and waits for every round trip.
+hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt) {
+  struct Tile {
+    int bm, bn, stages, occ;
+    double fixed, stage_lo, stage_hi;
+  };
+  static const Tile tiles[] = {{256, 256, 2, 1, 5.0, 1.10, 1.55},
+                               {256, 128, 3, 1, 4.0, 0.75, 0.93},
+                               {128, 128, 3, 1, 3.5, 0.45, 0.57},
+                               {128, 64, 4, 1, 3.3, 0.22, 0.36},
+                               {64, 64, 4, 2, 2.6, 0.19, 0.44}};
+  const double kt = static_cast<double>(ceil_div(K * elem_bytes(dt), 128));
+  constexpr double kCus = 256;
+  const Tile* best = nullptr;
+  double best_us = 0;
+  for (const Tile& t : tiles) {
+    const double n = static_cast<double>(ceil_div(M, t.bm)) * static_cast<double>(ceil_div(N, t.bn));
+    const double rounds = std::max(1.0, std::ceil(n / (kCus * t.occ)));
+    const double load = n / (rounds * kCus * t.occ);
+    const double us = rounds * (t.fixed + kt * (t.stage_lo + (t.stage_hi - t.stage_lo) * load));
+    if (!best || us < best_us) best = &t, best_us = us;
   }
-  // Small C: 64x64 tiles, or 32x32 tiles (one wave each) where 64x64 would
-  // occupy fewer than a quarter of the CUs: more workgroups share the
-  // latency of the K walk (f16 256^3, one box, back-to-back launches in a
-  // HIP graph: 3.11 us against 3.43 us).
-  const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
-  hxm_gemm_config c{64, 64, 0, 0, 0, 0, 1};
-  if (tiles64 < 64) c = hxm_gemm_config{32, 32, 0, 0, 0, 0, 1};
+  hxm_gemm_config c{best->bm, best->bn, 128 / elem_bytes(dt), 2, 2, best->stages, 1};
+  // Few small tiles of a short K: 32x32 tiles (one wave each), more workgroups
+  // to share the latency of the K walk (f16 256^3, one box, HIP graph: 3.11 us
+  // against 3.43 us for 64x64); from 20 stages on the deeper 64x64 tile wins
+  // (f16 100 x 256 x 8192 26.8 us against 28.8).
+  if (best->bm == 64 && ceil_div(M, 64) * ceil_div(N, 64) < 64 && kt < 20)
+    c = hxm_gemm_config{32, 32, 0, 0, 0, 0, 1};
   return kernel_config(static_cast<int>(find_kernel(c, dt) - kKernels), dt);
 }
 
@@ -284,7 +307,7 @@ hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64
     p->source = HXM_SOURCE_TUNED;
   } else {
     c = epi == kEpiFloat && small_gemm_fits(M, N, K, table) ? small_gemm_config()
-                                                             : default_config(M, N, table);
+                                                             : default_config(M, N, K, table);
     p->source = HXM_SOURCE_DEFAULT;
   }
   p->config = c;

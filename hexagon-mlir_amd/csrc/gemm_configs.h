@@ -4,7 +4,8 @@
 // this list; the LDS footprint is STAGES * (BM + BN) * BKB bytes.  The two
 // large tiles also come with a second wave grid (8 waves of 128x64, and 4x1
 // waves of 64x128), listed after the 2x2 grid that a lookup with wildcard
-// wave fields finds first.
+// wave fields finds first; the small tiles with a deeper prefetch (the
+// defaults of their sizes) after those with two stages for the same reason.
 #pragma once
 
 // A build may predefine the list (for example to compile one configuration).
@@ -14,7 +15,8 @@
       X(256, 128, 128, 3, 2, 2), X(256, 128, 64, 4, 2, 2),                       \
       X(128, 256, 64, 4, 2, 2), X(128, 128, 128, 2, 2, 2),                       \
       X(128, 128, 64, 4, 2, 2), X(64, 64, 128, 2, 2, 2), X(32, 32, 128, 2, 1, 1), \
-      X(256, 256, 128, 2, 2, 4), X(256, 128, 128, 3, 4, 1)
+      X(256, 256, 128, 2, 2, 4), X(256, 128, 128, 3, 4, 1),                      \
+      X(128, 128, 128, 3, 2, 2), X(128, 64, 128, 4, 2, 2), X(64, 64, 128, 4, 2, 2)
 #endif
 
 // W8A16 GEMM (f16 activations x int8 [N, K] weights, BKB = A bytes per
