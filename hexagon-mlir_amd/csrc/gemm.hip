@@ -307,6 +307,7 @@ hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64
     p->source = HXM_SOURCE_TUNED;
   } else {
     c = epi == kEpiFloat && small_gemm_fits(M, N, K, table) ? small_gemm_config()
+        : skinny_default(table, epi, M, N, K)                 ? skinny_config()
                                                              : default_config(M, N, K, table);
     p->source = HXM_SOURCE_DEFAULT;
   }
@@ -338,6 +339,22 @@ hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64
     return st;
   }
   hxm_status st = HXM_OK;
+  if (is_skinny_config(c)) {
+    if (!skinny_fits(M, N, K)) {
+      snprintf(why, sizeof(why), "the skinny kernel takes 1 to %lld rows and K > 0",
+               (long long)kSkinnyRowsMax);
+      st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_NO_KERNEL, why);
+    } else {
+      skinny_plan(table, epi, M, N, p);
+      p->workspace_bytes = extra_ws + (b_layout == HXM_B_KN ? N * kn_image_ld(K, eb) * eb : 0);
+      const bool full = M % 32 == 0 && N % 32 == 0 && K % 32 == 0;
+      p->plan = full ? HXM_PLAN_MFMA_FULL : HXM_PLAN_MFMA_TAIL;
+      p->reason = full ? HXM_REASON_SELECTED_ALIGNED : HXM_REASON_SELECTED_TAIL;
+    }
+    g_last_plan = *p;
+    if (entry) *entry = nullptr;
+    return st;
+  }
   const KernelEntry* e = find_kernel(c, table);
   if (!e) {
     snprintf(why, sizeof(why), "no compiled GEMM for bm=%d bn=%d bk=%d waves=%dx%d stages=%d",
@@ -407,7 +424,7 @@ static hxm_status run_gemm_with(int32_t op, int32_t ab_dtype, int epi, const voi
   int64_t ldb_bytes = 0;
   if (K > 0 && (st = resolve_b(B, ldb, b_layout, K, N, eb, stream, &bk, &ldb_bytes)) != HXM_OK)
     return st;
-  if (!e) {  // the plan chose the direct-load small-output kernel
+  if (!e && !is_skinny_config(plan.config)) {  // the direct-load small-output kernel
     if ((st = launch_small_gemm(ab_dtype, A, lda, bk, ldb_bytes, C, ldc, M, N, K, out_dtype,
                                 accumulate, stream)) != HXM_OK)
       return st;
@@ -436,6 +453,10 @@ static hxm_status run_gemm_with(int32_t op, int32_t ab_dtype, int epi, const voi
     const int64_t ob = dtype_bytes(out_dtype);
     g.vec_store = (reinterpret_cast<uintptr_t>(C) % (4 * ob) == 0) && ((ldc * ob) % (4 * ob) == 0);
     g.vec8_store = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && ((ldc * ob) % 16 == 0);
+  }
+  if (!e) {  // the plan chose the skinny kernel
+    if ((st = launch_skinny(ab_dtype, epi, g, stream)) != HXM_OK) return st;
+    return ok();
   }
   if (plan.k_slices > 1) {
     // K in S slices of whole stages (the plan's split); workgroup row z
@@ -618,7 +639,7 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
   } else if (lookup_tuned(op, M, sw ? n_out : N, K, &c)) {
     p->source = HXM_SOURCE_TUNED;
   } else {
-    c = skinny_fits(M, n_out, K) ? skinny_config() : default_w8_config(M, N, sw);
+    c = skinny_default(kSkinnyW8, epi, M, n_out, K) ? skinny_config() : default_w8_config(M, N, sw);
     p->source = HXM_SOURCE_DEFAULT;
   }
   p->config = c;
@@ -631,7 +652,7 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
                (long long)kSkinnyRowsMax);
       st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_NO_KERNEL, why);
     } else {
-      skinny_plan_w8(epi, M, n_out, p);
+      skinny_plan(kSkinnyW8, epi, M, n_out, p);
       const bool full = M % 32 == 0 && n_out % 32 == 0 && K % 32 == 0;
       p->plan = full ? HXM_PLAN_MFMA_FULL : HXM_PLAN_MFMA_TAIL;
       p->reason = full ? HXM_REASON_SELECTED_ALIGNED : HXM_REASON_SELECTED_TAIL;
@@ -721,7 +742,7 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
   g.vec_store = (reinterpret_cast<uintptr_t>(C) % 8 == 0) && ((ldc * 2) % 8 == 0);
   g.vec8_store = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && ((ldc * 2) % 16 == 0);
   if (!e) {  // the plan chose the skinny kernel
-    if ((st = launch_skinny_w8(epi, g, stream)) != HXM_OK) return st;
+    if ((st = launch_skinny(kSkinnyW8, epi, g, stream)) != HXM_OK) return st;
     return ok();
   }
   const int wi = static_cast<int>(e - kW8Kernels);

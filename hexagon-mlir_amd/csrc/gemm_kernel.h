@@ -61,13 +61,14 @@ enum Epilogue {
   kEpiFloat = 2,    // f16/bf16: fp32 acc -> out dtype (accumulate honoured)
   kEpiW8 = 3,       // f16 A x int8 B: f16(acc * cs[n])
   kEpiSwiglu = 4,   // f16 A x int8 gate/up image: f16(silu(g * sg) * (u * su))
-  kEpiW8Res = 5     // f16 A x int8 B: f16((acc * cs[n]) + r[m, n]), fp32 sum
+  kEpiW8Res = 5,    // f16 A x int8 B: f16((acc * cs[n]) + r[m, n]), fp32 sum
+  kEpiGemv = 6      // f16 A x int8 B: f16(acc * cs16[n]), f16 scales (skinny only)
 };
 
 // The int8-weight epilogues take B as int8 [N, K] converted to f16 in
 // registers (the W8A16 GEMM of the SwiGLU FFN).
 constexpr bool b_is_int8(int epi) {
-  return epi == kEpiW8 || epi == kEpiSwiglu || epi == kEpiW8Res;
+  return epi == kEpiW8 || epi == kEpiSwiglu || epi == kEpiW8Res || epi == kEpiGemv;
 }
 // The SwiGLU image (built by this library, never by the caller) stores each
 // weight in offset binary, byte = w + 128 (w ^ 0x80 as a bit pattern): that
@@ -1303,10 +1304,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
 
 typedef void (*gemm_fn)(GemmArgs);
 
-// The skinny W8A16 matmul (gemm_skinny.hip): fills a plan's config, threads,
-// tiles and LDS; launches (g as for the tile kernels).
-void skinny_plan_w8(int epi, int64_t M, int64_t n_out, hxm_plan* p);
-hxm_status launch_skinny_w8(int epi, const GemmArgs& g, hipStream_t stream);
+// The skinny matmul (gemm_skinny.hip): fills a plan's config, threads, tiles
+// and LDS; launches (g as for the tile kernels; n_out the output columns).
+void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, hxm_plan* p);
+hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, hipStream_t stream);
 
 // The compiled kernels.  Each kernel source (gemm_i8.hip, gemm_f16.hip,
 // gemm_w8.hip) is compiled kGemmParts times with HXM_PART = 0 .. kGemmParts-1

@@ -1,5 +1,6 @@
-// Launch rules of the skinny W8A16 matmuls (skinny_kernel.h): the default of
-// hxm_gemm_w8a16, _residual and _swiglu at 1 to kSkinnyRowsMax rows.
+// Launch rules of the skinny matmuls (skinny_kernel.h): the default of the
+// W8A16 GEMMs, of hxm_gemm_i8 / _dequant and of hxm_matmul at 1 to
+// kSkinnyRowsMax rows, and of hxm_gemv_w8a16 on plain [N, K] weights at 2 to 16.
 #include "skinny_kernel.h"
 
 namespace hxm {
@@ -7,48 +8,57 @@ namespace hxm {
 namespace {
 
 struct SkinnyShape {
-  int rows, groups, threads, lds;  // rows of A and 16-channel groups per workgroup
+  int rows, groups, threads, lds;  // rows of A and 16-channel output groups per workgroup
   void (*fn)(SkinnyArgs);
 };
 
-template <int MR, int CB, int NW, int SL, int U, int EPI>
-constexpr SkinnyShape w8_shape() {
-  constexpr int slab = CB * 16 * (SL + 16) +
-                       ((MR * SL * 2 / 16 + 63) / 64) * 64 / (SL * 2 / 16) * (SL * 2 + 16);
+template <int KIND, int MR, int CB, int NW, int SL, int U, int EPI>
+constexpr SkinnyShape shape() {
+  constexpr int al = SL * (KIND == kSkW8 ? 2 : 1) / 16;  // lanes per A row of a slab
+  constexpr int slab = CB * 16 * (SL + 16) + (MR * al + 63) / 64 * 64 / al * (al * 16 + 16);
   constexpr int mt = (MR + 15) / 16, mc = mt * CB <= 4 ? mt : (4 / CB > 0 ? 4 / CB : 1);
   constexpr int red = NW * mc * CB * 64 * 16, stg = NW * U * slab;
   return SkinnyShape{MR, EPI == kEpiSwiglu ? CB / 2 : CB, NW * 64, red > stg ? red : stg,
-                     skinny_kernel<kSkW8, MR, CB, NW, SL, U, EPI>};
+                     skinny_kernel<KIND, MR, CB, NW, SL, U, EPI>};
 }
 
 // The workgroup for M rows.  A rows are covered by the smallest of 4, 16, 32
 // and 64: rows past M cost no memory, but their LDS reads and MFMAs do run.
-// 128-byte slabs except at 64 rows, where a slab's A rows (16 KiB a wave)
-// would leave one wave per SIMD (gate/up 51.4 us against 40.7, down 35.5
-// against 30.4).  Gate/up takes 16 + 16 channels, the others 16: more
-// channels per workgroup share the A slabs but leave CUs idle (down, 16 rows:
-// 32 channels 22.0 us against 16.2 in 64-byte slabs).  Four waves instead of
-// eight from 32 rows up for gate/up, whose 688 workgroups fill the chip by
-// themselves.
-template <int EPI>
-SkinnyShape w8_shape_for(int64_t M) {
+// 128-byte slabs except for f16 x int8 at 64 rows, where a slab's A rows
+// (16 KiB a wave) would leave one wave per SIMD (gate/up 51.4 us against
+// 40.7, down 35.5 against 30.4).  Gate/up takes 16 + 16 channels, the others
+// 16: more channels per workgroup share the A slabs but leave CUs idle (down,
+// 16 rows: 32 channels 22.0 us against 16.2 in 64-byte slabs).  Four waves
+// instead of eight from 32 rows up for gate/up, whose 688 workgroups fill the
+// chip by themselves.
+template <int KIND, int EPI>
+SkinnyShape shape_for(int64_t M) {
   if constexpr (EPI == kEpiSwiglu) {
-    if (M <= 4) return w8_shape<4, 2, 8, 128, 1, EPI>();
-    if (M <= 16) return w8_shape<16, 2, 8, 128, 1, EPI>();
-    if (M <= 32) return w8_shape<32, 2, 4, 128, 1, EPI>();
-    return w8_shape<64, 2, 4, 64, 1, EPI>();
+    if (M <= 4) return shape<KIND, 4, 2, 8, 128, 1, EPI>();
+    if (M <= 16) return shape<KIND, 16, 2, 8, 128, 1, EPI>();
+    if (M <= 32) return shape<KIND, 32, 2, 4, 128, 1, EPI>();
+    return shape<KIND, 64, 2, 4, 64, 1, EPI>();
   } else {
-    if (M <= 4) return w8_shape<4, 1, 8, 128, 2, EPI>();
-    if (M <= 16) return w8_shape<16, 1, 8, 128, 1, EPI>();
-    if (M <= 32) return w8_shape<32, 1, 8, 128, 1, EPI>();
-    return w8_shape<64, 1, 8, 64, 1, EPI>();
+    if (M <= 4) return shape<KIND, 4, 1, 8, 128, 2, EPI>();
+    if (M <= 16 || EPI == kEpiGemv) return shape<KIND, 16, 1, 8, 128, 1, EPI>();
+    if constexpr (EPI != kEpiGemv) {
+      if (M <= 32) return shape<KIND, 32, 1, 8, 128, 1, EPI>();
+      return shape<KIND, 64, 1, 8, KIND == kSkW8 ? 64 : 128, 1, EPI>();
+    }
   }
 }
 
-SkinnyShape w8_shape_of(int epi, int64_t M) {
-  return epi == kEpiSwiglu  ? w8_shape_for<kEpiSwiglu>(M)
-         : epi == kEpiW8Res ? w8_shape_for<kEpiW8Res>(M)
-                            : w8_shape_for<kEpiW8>(M);
+SkinnyShape shape_of(int32_t table, int epi, int64_t M) {
+  switch (epi) {
+    case kEpiSwiglu: return shape_for<kSkW8, kEpiSwiglu>(M);
+    case kEpiW8Res: return shape_for<kSkW8, kEpiW8Res>(M);
+    case kEpiW8: return shape_for<kSkW8, kEpiW8>(M);
+    case kEpiGemv: return shape_for<kSkW8, kEpiGemv>(M);
+    case kEpiI32: return shape_for<kSkI8, kEpiI32>(M);
+    case kEpiDequant: return shape_for<kSkI8, kEpiDequant>(M);
+    default:
+      return table == HXM_BF16 ? shape_for<kSkBF16, kEpiFloat>(M) : shape_for<kSkF16, kEpiFloat>(M);
+  }
 }
 
 int64_t groups_of(const SkinnyShape& s, int64_t n_out) {
@@ -69,15 +79,35 @@ bool skinny_fits(int64_t M, int64_t N, int64_t K) {
   return M > 0 && N > 0 && K > 0 && M <= kSkinnyRowsMax && grid_fits((N + 15) / 16, 512);
 }
 
-void skinny_plan_w8(int epi, int64_t M, int64_t n_out, hxm_plan* p) {
-  const SkinnyShape s = w8_shape_of(epi, M);
+// Up to 32 rows the skinny kernel streams the weights faster than any tile.
+// Above, a workgroup of 16 channels x 64 rows pays for its own A slabs, and the
+// line is drawn by how many of them the chip must run (f16, N x K, M: skinny /
+// best tile us, HIP graph, one box): 4096 x 4096, 64: 13.2 / 14.4 (256
+// workgroups); 1024 x 4096, 256: 11.2 / 14.0 (256); 2048 x 4096, 192: 19.3 /
+// 14.4 (384); below 2 KiB of K the tiles' fixed time is the shorter one (4096 x
+// 512, 64: 4.4 / 4.1). int8 alike. f16 x int8 against its 128-row tiles,
+// down projection 4096 x 2048: 64 rows 7.1 / 16.1 (256), 128 12.8 / 16.2 (512),
+// 192 17.9 / 16.4 (768); gate/up 2048 x 4096: 256 rows 23.9 / 40.7 (512),
+// 11008 x 4096: 64 rows 42.1 / 41.2 (688), 96 70.8 / 41.8 (1376).
+bool skinny_default(int32_t table, int epi, int64_t M, int64_t n_out, int64_t K) {
+  if (!skinny_fits(M, n_out, K)) return false;
+  const int64_t kb = table == kSkinnyW8 ? K : K * dtype_bytes(table);
+  if (M <= 32) return table == kSkinnyW8 || kb >= 256;
+  const SkinnyShape s = shape_of(table, epi, M);
+  const int64_t groups = groups_of(s, n_out) * ((M + s.rows - 1) / s.rows);
+  if (table == kSkinnyW8) return groups <= (epi == kEpiSwiglu ? 700 : 512);
+  return kb >= 2048 && groups <= 256;
+}
+
+void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, hxm_plan* p) {
+  const SkinnyShape s = shape_of(table, epi, M);
   p->config = skinny_config();
   p->threads = s.threads;
   p->tiles = groups_of(s, n_out) * ((M + s.rows - 1) / s.rows);
   p->lds_bytes = s.lds;
 }
 
-hxm_status launch_skinny_w8(int epi, const GemmArgs& g, hipStream_t stream) {
+hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, hipStream_t stream) {
   SkinnyArgs a{};
   a.A = g.A;
   a.B = g.B;
@@ -87,16 +117,19 @@ hxm_status launch_skinny_w8(int epi, const GemmArgs& g, hipStream_t stream) {
   a.ldc = g.ldc;
   a.M = g.M;
   a.N = g.N;
-  a.KB = g.K_bytes / 2;
+  a.KB = table == kSkinnyW8 ? g.K_bytes / 2 : g.K_bytes;
   a.n_out = g.n_out;
+  a.out_dtype = g.out_dtype;
+  a.accumulate = g.accumulate;
+  a.row_scale = g.row_scale;
   a.col_scale = g.col_scale;
   a.residual = g.residual;
   a.ldr = g.ldr;
-  const SkinnyShape s = w8_shape_of(epi, g.M);
-  const dim3 grid(static_cast<unsigned>(groups_of(s, g.n_out)),
+  const SkinnyShape s = shape_of(table, epi, g.M);
+  const dim3 grid(static_cast<unsigned>(groups_of(s, epi == kEpiSwiglu ? g.n_out : g.N)),
                   static_cast<unsigned>((g.M + s.rows - 1) / s.rows));
   hipLaunchKernelGGL(s.fn, grid, dim3(s.threads), 0, stream, a);
-  return check_launch("skinny w8a16 gemm");
+  return check_launch("skinny gemm");
 }
 
 }  // namespace hxm

@@ -24,8 +24,7 @@
 //   * at M = 1 and with three channel groups per workgroup, the groups go to
 //     workgroups XCD-contiguously (gemv_block), so each XCD streams one
 //     contiguous eighth of the weight image.
-#include "device_util.h"
-#include "hxm_internal.h"
+#include "gemm_kernel.h"
 
 namespace hxm {
 
@@ -551,11 +550,31 @@ hxm_status hxm_gemv_w8a16(const void* x, int64_t ldx, const int8_t* W, int64_t l
     return check_launch("gemv_w8a16");
   }
   const bool pk = w_layout == HXM_W_PACKED;
-  // Channel groups per workgroup at M > 4: three share each staged x chunk,
-  // which pays while a workgroup per 16 channels would more than fill the
-  // chip; below that (fewer than kGemvCb3MinGroups groups, a column shard
-  // for example) the three-fold grid leaves CUs idle.
-  const int cb = M <= 4 || (N + 15) / 16 < kGemvCb3MinGroups ? 1 : 3;
+  // The plain [N, K] layout at M > 1 takes the skinny kernel, which reads whole
+  // lines of W where the kernels here read a 64-byte piece of each of 16 rows
+  // per instruction (one box, one-chunk kernel / skinny): M=16 N=4096 K=11008
+  // 17.7 / 13.3 us.  Its 32-bit offsets span 64 rows of at most 2^23 bytes.
+  constexpr int64_t kRowMax = int64_t(1) << 23;
+  if (!pk && M > 1 && ldw <= kRowMax && ldx * 2 <= kRowMax) {
+    if ((st = check_grid("gemv_w8a16", (N + 15) / 16, 512, (M + 15) / 16)) != HXM_OK) return st;
+    GemmArgs a{};
+    a.A = static_cast<const uint8_t*>(x);
+    a.B = reinterpret_cast<const uint8_t*>(W);
+    a.C = y;
+    a.lda_bytes = ldx * 2;
+    a.ldb_bytes = ldw;
+    a.ldc = ldy;
+    a.M = g.M;
+    a.N = g.N;
+    a.K_bytes = g.K * 2;
+    a.col_scale = static_cast<const float*>(w_scale);  // f16 values (kEpiGemv)
+    return launch_skinny(kSkinnyW8, kEpiGemv, a, s);
+  }
+  // Channel groups per workgroup at M > 4 (packed image): three share each
+  // staged x chunk, which pays while a workgroup per 16 channels would more
+  // than fill the chip; below that (fewer than kGemvCb3MinGroups groups, a
+  // column shard for example) the three-fold grid leaves CUs idle.
+  const int cb = !pk || M <= 4 || (N + 15) / 16 < kGemvCb3MinGroups ? 1 : 3;
   if ((st = check_grid("gemv_w8a16", (N + 16 * cb - 1) / (16 * cb), 512, (M + 15) / 16)) != HXM_OK)
     return st;
   // M = 1 (and the plain [N, K] layout at every M, and the packed image at
@@ -574,15 +593,14 @@ hxm_status hxm_gemv_w8a16(const void* x, int64_t ldx, const int8_t* W, int64_t l
       gemv_w8a16_pipe_kernel<8, 4, 1, true, false><<<grid(1), 512, 0, s>>>(g);
     else if (pk)
       gemv_w8a16_kernel<8, 8, true, 4, 1, true, false><<<grid(1), 512, 0, s>>>(g);
-    else
-      gemv_w8a16_kernel<8, 8, false, 4, 1, true, false><<<grid(1), 512, 0, s>>>(g);
+    else  // rows too far apart for the skinny kernel's offsets
+      gemv_w8a16_kernel<8, 4, false, 16, 1, false, false><<<grid(1), 512, 0, s>>>(g);
   } else {
     // 16 x rows: three channel groups per workgroup share each staged x
     // chunk (measured with the one-chunk kernel: 13.1 vs 14.7 us at
     // N=11008, K=4096), one group below kGemvCb3MinGroups.
     if (pk && cb == 3) gemv_w8a16_pipe_kernel<8, 16, 3, false, true><<<grid(3), 512, 0, s>>>(g);
     else if (pk) gemv_w8a16_pipe_kernel<8, 16, 1, false, false><<<grid(1), 512, 0, s>>>(g);
-    else if (cb == 3) gemv_w8a16_kernel<8, 4, false, 16, 3, false, true><<<grid(3), 512, 0, s>>>(g);
     else gemv_w8a16_kernel<8, 4, false, 16, 1, false, false><<<grid(1), 512, 0, s>>>(g);
   }
   return check_launch("gemv_w8a16");

@@ -103,9 +103,13 @@ hxm_status pack_f32_operands(const float* A, int64_t lda, _Float16* ai, int64_t 
                              int64_t ldb, _Float16* bi, int64_t N, int64_t K, int64_t kp, bool kn,
                              hipStream_t stream);
 
-// The skinny W8A16 matmul (gemm_skinny.hip): the default of the W8A16 GEMMs at
-// 1 to kSkinnyRowsMax rows; a caller names it with skinny_config().
-constexpr int64_t kSkinnyRowsMax = 64;
+// The skinny matmul (gemm_skinny.hip): takes 1 to kSkinnyRowsMax rows and is
+// the default where skinny_default says so (table: the operand dtype, or
+// kSkinnyW8 for f16 A and int8 B; epi: gemm_kernel.h's Epilogue); a caller names
+// it with skinny_config().
+constexpr int64_t kSkinnyRowsMax = 256;
+constexpr int32_t kSkinnyW8 = 0;
+bool skinny_default(int32_t table, int epi, int64_t M, int64_t n_out, int64_t K);
 hxm_gemm_config skinny_config();
 bool is_skinny_config(const hxm_gemm_config& c);
 bool skinny_fits(int64_t M, int64_t N, int64_t K);

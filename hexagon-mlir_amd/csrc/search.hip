@@ -816,8 +816,7 @@ hxm_status hxm_tune_cache_load(const char* path, int32_t* loaded) {
     // The small-output kernel is a winner only for shapes it takes.
     const bool small_ok = (op == HXM_F16 || op == HXM_BF16) && is_small_gemm_config(c) &&
                           small_gemm_fits(ent.m, ent.n, ent.k, op);
-    const bool skinny_ok = (op == HXM_OP_W8A16 || op == HXM_OP_W8A16_SWIGLU) &&
-                           is_skinny_config(c) && skinny_fits(ent.m, ent.n, ent.k);
+    const bool skinny_ok = is_skinny_config(c) && skinny_fits(ent.m, ent.n, ent.k);
     if (!small_ok && !skinny_ok && !config_compiled(op, c)) continue;
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[TuneKey(op, ent.m, ent.n, ent.k)] = c;
@@ -886,7 +885,10 @@ hxm_status hxm_tune_gemm(int32_t op, const void* A, int64_t lda, const void* B,
   const bool small = op != HXM_I8 && small_gemm_fits(M, N, K, op);
   if (small) sp.cands.push_back(small_gemm_config());
   sort_configs(&sp.cands);
-  sp.control = small ? small_gemm_config() : default_config(M, N, K, op);
+  sp.control = small ? small_gemm_config()
+               : skinny_default(op, epi, M, N, K) ? skinny_config()
+                                             : default_config(M, N, K, op);
+  if (skinny_fits(M, N, K)) sp.cands.insert(sp.cands.begin(), skinny_config());
   sp.canary = hxm_gemm_config{32, 32, static_cast<int32_t>(op == HXM_I8 ? 128 : 64), 1, 1, 2, 1};
   sp.cm = std::min<int64_t>(32, M), sp.cn = std::min<int64_t>(32, N);
   const int64_t ck = std::min<int64_t>(K, 32);
@@ -953,10 +955,8 @@ hxm_status hxm_tune_w8a16(int32_t op, const void* x, int64_t ldx, const int8_t* 
   sort_configs(&sp.cands);
   sp.control = default_w8_config(M, rows, sw);
   sp.canary = sp.cands.front();  // the smallest compiled tile on a 32-row slice
-  if (skinny_fits(M, N, K)) {    // what an untuned call runs
-    sp.control = skinny_config();
-    sp.cands.insert(sp.cands.begin(), sp.control);
-  }
+  if (skinny_fits(M, N, K)) sp.cands.insert(sp.cands.begin(), skinny_config());
+  if (skinny_default(kSkinnyW8, epi, M, N, K)) sp.control = skinny_config();
   sp.cm = std::min<int64_t>(32, M), sp.cn = std::min<int64_t>(sw ? 64 : 32, N);
   sp.ck = std::min<int64_t>(K, 32);
   sp.run = [=](const hxm_gemm_config& c, int64_t m, int64_t n, int64_t k) {

@@ -52,7 +52,7 @@ struct SkinnyArgs {
   int out_dtype;     // kEpiFloat: HXM_F16 / HXM_BF16 / HXM_F32
   int accumulate;    // kEpiI32, kEpiFloat
   const float* row_scale;
-  const float* col_scale;
+  const float* col_scale;    // kEpiGemv: f16
   const _Float16* residual;  // kEpiW8Res
   int64_t ldr;
 };
@@ -297,9 +297,12 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
             const float ex = __builtin_amdgcn_exp2f(-gv * 1.4426950408889634f);
             h[v] = static_cast<_Float16>(gv * __builtin_amdgcn_rcpf(1.0f + ex) * uv);
           } else {
-            float p = EPI == kEpiDequant
-                          ? (static_cast<float>(a[v]) * g.row_scale[m]) * g.col_scale[nv]
-                          : static_cast<float>(a[v]) * g.col_scale[nv];
+            float p = static_cast<float>(a[v]);
+            if constexpr (EPI == kEpiDequant) p *= g.row_scale[m];
+            if constexpr (EPI == kEpiGemv)
+              p *= static_cast<float>(reinterpret_cast<const _Float16*>(g.col_scale)[nv]);
+            else
+              p *= g.col_scale[nv];
             asm volatile("" : "+v"(p));
             if constexpr (EPI == kEpiW8Res) {
               p = p + static_cast<float>(g.residual[static_cast<int64_t>(m) * g.ldr + nv]);

@@ -213,7 +213,9 @@ int32_t hxm_last_plan(hxm_plan* out);
  * with K <= 256 runs on the direct-load small-output kernel (config
  * {16,16,32,1,1,0,1}, one wave per 16x16 tile, no LDS); the same config
  * passed in cfg asks for it and is refused (HXM_UNSUPPORTED_SHAPE,
- * "no-kernel") outside those limits. */
+ * "no-kernel") outside those limits.  Other outputs of few rows run on the
+ * skinny kernel of the W8A16 GEMMs (config {16,16,64,1,8,0,1}, 1 to 256 rows),
+ * as do those of hxm_gemm_i8 and hxm_gemm_i8_dequant. */
 hxm_status hxm_matmul(const void* A, int64_t lda, const void* B, int64_t ldb,
                       int32_t b_layout, void* C, int64_t ldc, int64_t M,
                       int64_t N, int64_t K, int32_t ab_dtype, int32_t c_dtype,
@@ -367,10 +369,11 @@ enum { HXM_OP_W8A16 = 16, HXM_OP_W8A16_SWIGLU = 17 };
  * multiple of 16, x and W 16-byte aligned, and 256 rows of x and of W
  * within 2 GiB (as for hxm_matmul).  cfg: NULL = tuned winner or the
  * default; else one of hxm_w8a16_configs.  With cfg NULL and no tuned winner,
- * 1 to 64 rows run on the skinny kernel (config {16,16,64,1,8,0,1}: the
+ * few rows (1 to 32, and up to 256 while the output has few enough 16-channel
+ * x 64-row blocks) run on the skinny kernel (config {16,16,64,1,8,0,1}: the
  * waves of a workgroup split K, partial sums added in a fixed order); the
  * same config passed in cfg asks for it and is refused
- * (HXM_UNSUPPORTED_SHAPE, "no-kernel") outside those limits. */
+ * (HXM_UNSUPPORTED_SHAPE, "no-kernel") above 256 rows. */
 hxm_status hxm_gemm_w8a16(const void* x, int64_t ldx, const int8_t* W,
                           int64_t ldw, const float* w_scale, void* y,
                           int64_t ldy, int64_t M, int64_t N, int64_t K,

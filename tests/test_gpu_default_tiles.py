@@ -18,7 +18,7 @@ def bits(t):
 
 
 # (M, N, K bytes, tile): K ends inside a stage; M and N inside a tile.
-SHAPES = [(70, 333, 2576, (64, 64)), (300, 4001, 1040, (64, 64)), (1001, 1500, 2576, (128, 64)),
+SHAPES = [(260, 333, 2576, (64, 64)), (300, 4001, 1040, (64, 64)), (1001, 1500, 2576, (128, 64)),
           (1990, 2010, 400, (128, 128)), (2041, 4072, 272, (256, 128))]
 
 

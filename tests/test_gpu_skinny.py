@@ -1,6 +1,6 @@
-"""The skinny matmul (csrc/skinny_kernel.h), the default of the W8A16 GEMMs at 1 to 64
+"""The skinny matmul (csrc/skinny_kernel.h), the default of the matmuls of few
 rows, against the CPU oracle: at the edges of its row blocks (4, 16, 32,
-64), with channels and K that end inside a group, a slab and a 64-byte piece
+64, several of 64), with channels and K that end inside a group, a slab and a 64-byte piece
 of one.  Operands are views of wider buffers whose padding holds NaN (x) or
 127 (W), so a chunk read past K or M would show, and the output's padding
 must keep its fill."""
@@ -32,7 +32,7 @@ def padded(t, fill, dev, rows=3, cols=16):
     return buf, v
 
 
-@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 64, 65, 256])
 @pytest.mark.parametrize("N,K", [(8, 16), (100, 112), (333, 656), (272, 2064)])
 def test_w8a16_and_residual(dev, M, N, K):
     print(f"skinny w8a16 M={M} N={N} K={K}", flush=True)
@@ -55,7 +55,7 @@ def test_w8a16_and_residual(dev, M, N, K):
     np.testing.assert_allclose(z.float().cpu().numpy(), ref, **TOL)
 
 
-@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 64, 150])
 @pytest.mark.parametrize("I,K", [(16, 16), (100, 656), (200, 1040)])
 def test_swiglu(dev, M, I, K):
     print(f"skinny swiglu M={M} I={I} K={K}", flush=True)
@@ -99,11 +99,11 @@ def test_exact_sums_match_the_tiles_bit_for_bit(dev, M):
 
 
 def test_named_config_and_tuner(dev):
-    x = torch.randn(65, 64, device=dev).half()
+    x = torch.randn(257, 64, device=dev).half()
     W = torch.ones(32, 64, dtype=torch.int8, device=dev)
     s = torch.ones(32, device=dev)
     with pytest.raises(hxm.HxmError, match="no-kernel"):
-        ops.gemm_w8a16(x, W, s, config=SKINNY)           # 65 rows
+        ops.gemm_w8a16(x, W, s, config=SKINNY)           # 257 rows
     y = ops.gemm_w8a16(x[:64], W, s, config=SKINNY)
     assert ops.last_plan()["source"] == "caller"
     hxm.lib.hxm_tune_cache_clear()
@@ -112,3 +112,70 @@ def test_named_config_and_tuner(dev):
     assert ctl["tiles"] == [16, 16, 64] and ctl["stages"] == 0
     assert all(c["verified"] for c in rep["configs"] if c["q50"] is not None)
     hxm.lib.hxm_tune_cache_clear()
+
+
+@pytest.mark.parametrize("M", [1, 5, 17, 32, 33, 64, 100])
+@pytest.mark.parametrize("N,K", [(8, 2048), (333, 2064), (40, 272)])
+def test_int8(dev, M, N, K):
+    """int32 (plain and accumulated) and dequant outputs, bit for bit."""
+    print(f"skinny int8 M={M} N={N} K={K}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    B = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    _, Ad = padded(A, 111, dev)
+    _, Bd = padded(B, 111, dev)
+    ref = orc.gemm_i8(A.numpy(), B.numpy(), b_nk=True)
+    C0 = torch.randint(-1000, 1000, (M, N), generator=g, dtype=torch.int32)
+    cbuf, c = padded(C0, 7, dev)
+    ops.gemm_i8(Ad, Bd, out=c, b_layout="nk", config=SKINNY)
+    assert np.array_equal(c.cpu().numpy(), ref)
+    c.copy_(C0)
+    ops.gemm_i8(Ad, Bd, out=c, b_layout="nk", accumulate=True, config=SKINNY)
+    assert np.array_equal(c.cpu().numpy(), ref + C0.numpy())
+    assert (cbuf[:, N:] == 7).all() and (cbuf[M:] == 7).all()
+    rs, cs = (torch.rand(n, generator=g) * 0.019 + 0.001 for n in (M, N))
+    D = ops.gemm_i8_dequant(Ad, Bd, rs.to(dev), cs.to(dev), b_layout="nk", config=SKINNY)
+    assert np.array_equal(bits(D), orc.dequant_f16(ref, rs.numpy(), cs.numpy()))
+
+
+@pytest.mark.parametrize("M", [1, 5, 17, 32, 33, 64, 100])
+@pytest.mark.parametrize("N,K", [(8, 1024), (333, 1032), (40, 136)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_float(dev, dt, M, N, K):
+    """f16 / bf16 operands into f32 (accumulated too) and their own dtype; the
+    padding of A and B is NaN."""
+    print(f"skinny {dt} M={M} N={N} K={K}", flush=True)
+    name = "f16" if dt == torch.float16 else "bf16"
+    g = torch.Generator().manual_seed(M + N + K)
+    A = (torch.rand(M, K, generator=g) * 2 - 1).to(dt)
+    B = (torch.rand(N, K, generator=g) * 2 - 1).to(dt)
+    _, Ad = padded(A, float("nan"), dev)
+    _, Bd = padded(B, float("nan"), dev)
+    C0 = torch.randn(M, N, generator=g)
+    ref = orc.matmul(bits(A), bits(B), ab_dtype=name, c_dtype="f32", b_nk=True)
+    cbuf, c = padded(C0, 7.0, dev)
+    ops.matmul(Ad, Bd, out=c, b_layout="nk", config=SKINNY)
+    np.testing.assert_allclose(c.cpu().numpy(), ref, rtol=1e-4, atol=1e-4)
+    c.copy_(C0)
+    ops.matmul(Ad, Bd, out=c, b_layout="nk", accumulate=True, config=SKINNY)
+    np.testing.assert_allclose(c.cpu().numpy(), ref + C0.numpy(), rtol=1e-4, atol=1e-4)
+    assert (cbuf[:, N:] == 7).all() and (cbuf[M:] == 7).all()
+    h = ops.matmul(Ad, Bd, b_layout="nk", config=SKINNY)
+    np.testing.assert_allclose(h.float().cpu().numpy(), ref, rtol=1e-2, atol=1e-3)
+
+
+@pytest.mark.parametrize("M", [2, 4, 5, 16, 17, 40])
+@pytest.mark.parametrize("N,K", [(40, 16), (333, 656), (100, 2064)])
+def test_gemv_plain_weights(dev, M, N, K):
+    print(f"skinny gemv M={M} N={N} K={K}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).half()
+    W = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    s = (torch.rand(N, generator=g) * 0.019 + 0.001).half()
+    _, xd = padded(x, float("nan"), dev)
+    _, Wd = padded(W, 127, dev)
+    ybuf, y = padded(torch.zeros(M, N).half(), 7.0, dev)
+    ops.gemv_w8a16(xd, Wd, s.to(dev), out=y)
+    ref = orc.f16_bits_to_f32(orc.gemv_w8a16(bits(x), W.numpy(), bits(s)))
+    np.testing.assert_allclose(y.float().cpu().numpy(), ref, **TOL)
+    assert (ybuf[:, N:] == 7).all() and (ybuf[M:] == 7).all()
