@@ -106,4 +106,32 @@ __device__ __forceinline__ v8f16 i8x8_to_f16(uint32_t lo, uint32_t hi) {
   return __builtin_bit_cast(v8f16, r);
 }
 
+// 16 bytes of K (from row k of an LDS tile [K][pitch bytes], pitch a multiple of
+// 4) at byte column `col`: EB-byte elements of neighbouring rows picked out of
+// the words that hold them.
+template <int EB>
+__device__ __forceinline__ v4i32 kn_fragment(const uint8_t* tile, int pitch, int k, int col) {
+  constexpr int E = 16 / EB;
+  uint32_t d[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    d[e] = *reinterpret_cast<const uint32_t*>(tile + (k + e) * pitch + (col & ~3));
+  v4i32 r;
+  if constexpr (EB == 2) {
+    const uint32_t sel = col & 2 ? 0x07060302u : 0x05040100u;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      r[w] = static_cast<int>(__builtin_amdgcn_perm(d[2 * w + 1], d[2 * w], sel));
+  } else {
+    const uint32_t sel = static_cast<uint32_t>(col & 3) * 0x0101u + 0x0400u;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t lo = __builtin_amdgcn_perm(d[4 * w + 1], d[4 * w], sel);
+      const uint32_t hi = __builtin_amdgcn_perm(d[4 * w + 3], d[4 * w + 2], sel);
+      r[w] = static_cast<int>(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
+    }
+  }
+  return r;
+}
+
 }  // namespace hxm

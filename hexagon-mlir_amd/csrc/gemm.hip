@@ -345,8 +345,10 @@ hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64
                (long long)kSkinnyRowsMax);
       st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_NO_KERNEL, why);
     } else {
-      skinny_plan(table, epi, M, N, p);
-      p->workspace_bytes = extra_ws + (b_layout == HXM_B_KN ? N * kn_image_ld(K, eb) * eb : 0);
+      const bool direct = b_layout == HXM_B_KN && skinny_takes_kn(N, K, eb);  // read as it is
+      skinny_plan(table, epi, M, N, direct, p);
+      p->workspace_bytes =
+          extra_ws + (b_layout == HXM_B_KN && !direct ? N * kn_image_ld(K, eb) * eb : 0);
       const bool full = M % 32 == 0 && N % 32 == 0 && K % 32 == 0;
       p->plan = full ? HXM_PLAN_MFMA_FULL : HXM_PLAN_MFMA_TAIL;
       p->reason = full ? HXM_REASON_SELECTED_ALIGNED : HXM_REASON_SELECTED_TAIL;
@@ -422,11 +424,20 @@ static hxm_status run_gemm_with(int32_t op, int32_t ab_dtype, int epi, const voi
   if (M == 0 || N == 0) return ok();
   const uint8_t* bk = nullptr;
   int64_t ldb_bytes = 0;
-  if (K > 0 && (st = resolve_b(B, ldb, b_layout, K, N, eb, stream, &bk, &ldb_bytes)) != HXM_OK)
+  // The small-output and skinny kernels read a [K, N] B as it is.
+  const bool small = !e && !is_skinny_config(plan.config);
+  const bool direct = b_layout == HXM_B_KN && !e &&
+                      (small ? small_takes_kn(N) : skinny_takes_kn(N, K, eb));
+  if (direct) {
+    bk = static_cast<const uint8_t*>(B);
+    ldb_bytes = ldb * eb;
+  } else if (K > 0 && (st = resolve_b(B, ldb, b_layout, K, N, eb, stream, &bk, &ldb_bytes)) !=
+                          HXM_OK) {
     return st;
-  if (!e && !is_skinny_config(plan.config)) {  // the direct-load small-output kernel
-    if ((st = launch_small_gemm(ab_dtype, A, lda, bk, ldb_bytes, C, ldc, M, N, K, out_dtype,
-                                accumulate, stream)) != HXM_OK)
+  }
+  if (small) {  // the plan chose the direct-load small-output kernel
+    if ((st = launch_small_gemm(ab_dtype, A, lda, bk, ldb_bytes, direct, C, ldc, M, N, K,
+                                out_dtype, accumulate, stream)) != HXM_OK)
       return st;
     return ok();
   }
@@ -455,7 +466,7 @@ static hxm_status run_gemm_with(int32_t op, int32_t ab_dtype, int epi, const voi
     g.vec8_store = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && ((ldc * ob) % 16 == 0);
   }
   if (!e) {  // the plan chose the skinny kernel
-    if ((st = launch_skinny(ab_dtype, epi, g, stream)) != HXM_OK) return st;
+    if ((st = launch_skinny(ab_dtype, epi, g, direct, stream)) != HXM_OK) return st;
     return ok();
   }
   if (plan.k_slices > 1) {
@@ -652,7 +663,7 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
                (long long)kSkinnyRowsMax);
       st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_NO_KERNEL, why);
     } else {
-      skinny_plan(kSkinnyW8, epi, M, n_out, p);
+      skinny_plan(kSkinnyW8, epi, M, n_out, false, p);
       const bool full = M % 32 == 0 && n_out % 32 == 0 && K % 32 == 0;
       p->plan = full ? HXM_PLAN_MFMA_FULL : HXM_PLAN_MFMA_TAIL;
       p->reason = full ? HXM_REASON_SELECTED_ALIGNED : HXM_REASON_SELECTED_TAIL;
@@ -742,7 +753,7 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
   g.vec_store = (reinterpret_cast<uintptr_t>(C) % 8 == 0) && ((ldc * 2) % 8 == 0);
   g.vec8_store = (reinterpret_cast<uintptr_t>(C) % 16 == 0) && ((ldc * 2) % 16 == 0);
   if (!e) {  // the plan chose the skinny kernel
-    if ((st = launch_skinny(kSkinnyW8, epi, g, stream)) != HXM_OK) return st;
+    if ((st = launch_skinny(kSkinnyW8, epi, g, false, stream)) != HXM_OK) return st;
     return ok();
   }
   const int wi = static_cast<int>(e - kW8Kernels);

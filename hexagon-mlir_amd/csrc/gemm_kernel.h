@@ -1306,8 +1306,10 @@ typedef void (*gemm_fn)(GemmArgs);
 
 // The skinny matmul (gemm_skinny.hip): fills a plan's config, threads, tiles
 // and LDS; launches (g as for the tile kernels; n_out the output columns).
-void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, hxm_plan* p);
-hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, hipStream_t stream);
+// kn: B is the plain [K, N] operand, rows of ldb_bytes (where skinny_takes_kn).
+bool skinny_takes_kn(int64_t N, int64_t K, int64_t elem_bytes);
+void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, bool kn, hxm_plan* p);
+hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, bool kn, hipStream_t stream);
 
 // The compiled kernels.  Each kernel source (gemm_i8.hip, gemm_f16.hip,
 // gemm_w8.hip) is compiled kGemmParts times with HXM_PART = 0 .. kGemmParts-1

@@ -12,14 +12,15 @@ struct SkinnyShape {
   void (*fn)(SkinnyArgs);
 };
 
-template <int KIND, int MR, int CB, int NW, int SL, int U, int EPI>
+template <int KIND, int MR, int CB, int NW, int SL, int U, int EPI, bool KN = false>
 constexpr SkinnyShape shape() {
   constexpr int al = SL * (KIND == kSkW8 ? 2 : 1) / 16;  // lanes per A row of a slab
-  constexpr int slab = CB * 16 * (SL + 16) + (MR * al + 63) / 64 * 64 / al * (al * 16 + 16);
+  constexpr int eb = KIND == kSkF16 || KIND == kSkBF16 ? 2 : 1;
+  constexpr int slab = (KN ? SL / eb * (16 * CB * eb + 4) : CB * 16 * (SL + 16)) + (MR * al + 63) / 64 * 64 / al * (al * 16 + 16);
   constexpr int mt = (MR + 15) / 16, mc = mt * CB <= 4 ? mt : (4 / CB > 0 ? 4 / CB : 1);
   constexpr int red = NW * mc * CB * 64 * 16, stg = NW * U * slab;
   return SkinnyShape{MR, EPI == kEpiSwiglu ? CB / 2 : CB, NW * 64, red > stg ? red : stg,
-                     skinny_kernel<KIND, MR, CB, NW, SL, U, EPI>};
+                     skinny_kernel<KIND, MR, CB, NW, SL, U, EPI, KN>};
 }
 
 // The workgroup for M rows.  A rows are covered by the smallest of 4, 16, 32
@@ -61,6 +62,23 @@ SkinnyShape shape_of(int32_t table, int epi, int64_t M) {
   }
 }
 
+// A [K, N] B: 32 channels per workgroup (64 or 32 bytes of each row; with 16 a
+// row piece would be a quarter of a line or less), one batch ahead.
+template <int KIND, int EPI>
+SkinnyShape kn_shape_for(int64_t M) {
+  if (M <= 4) return shape<KIND, 4, 2, 8, 128, 1, EPI, true>();
+  if (M <= 16) return shape<KIND, 16, 2, 8, 128, 1, EPI, true>();
+  if (M <= 32) return shape<KIND, 32, 2, 8, 128, 1, EPI, true>();
+  return shape<KIND, 64, 2, 8, 128, 1, EPI, true>();
+}
+
+SkinnyShape kn_shape_of(int32_t table, int epi, int64_t M) {
+  if (epi == kEpiI32) return kn_shape_for<kSkI8, kEpiI32>(M);
+  if (epi == kEpiDequant) return kn_shape_for<kSkI8, kEpiDequant>(M);
+  return table == HXM_BF16 ? kn_shape_for<kSkBF16, kEpiFloat>(M)
+                           : kn_shape_for<kSkF16, kEpiFloat>(M);
+}
+
 int64_t groups_of(const SkinnyShape& s, int64_t n_out) {
   return ((n_out + 15) / 16 + s.groups - 1) / s.groups;
 }
@@ -99,15 +117,25 @@ bool skinny_default(int32_t table, int epi, int64_t M, int64_t n_out, int64_t K)
   return kb >= 2048 && groups <= 256;
 }
 
-void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, hxm_plan* p) {
-  const SkinnyShape s = shape_of(table, epi, M);
+void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, bool kn, hxm_plan* p) {
+  const SkinnyShape s = kn ? kn_shape_of(table, epi, M) : shape_of(table, epi, M);
   p->config = skinny_config();
   p->threads = s.threads;
   p->tiles = groups_of(s, n_out) * ((M + s.rows - 1) / s.rows);
   p->lds_bytes = s.lds;
 }
 
-hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, hipStream_t stream) {
+// Reading B once instead of packing it first (read, write, read): f16 direct /
+// pack and skinny / pack and best tile (us, HIP graph, one box), 16 rows: 512 x
+// 512 3.3 / 4.6 / 6.3, 2048 x 2048 5.7 / 11.4 / 14.5, 4096 x 4096 11.5 / 19.6 /
+// 25.6; int8 4096 x 4096 7.9 / 16.7 / 19.7.  Few workgroups with a long K are
+// the exception, which the pack spreads over the chip: 512 x 4096 8.7 / 7.5,
+// 64 x 8192 14.6 / 11.8.
+bool skinny_takes_kn(int64_t N, int64_t K, int64_t elem_bytes) {
+  return N * elem_bytes >= 16 && !((N + 31) / 32 <= 16 && K * elem_bytes >= 8192);
+}
+
+hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, bool kn, hipStream_t stream) {
   SkinnyArgs a{};
   a.A = g.A;
   a.B = g.B;
@@ -125,7 +153,7 @@ hxm_status launch_skinny(int32_t table, int epi, const GemmArgs& g, hipStream_t 
   a.col_scale = g.col_scale;
   a.residual = g.residual;
   a.ldr = g.ldr;
-  const SkinnyShape s = shape_of(table, epi, g.M);
+  const SkinnyShape s = kn ? kn_shape_of(table, epi, g.M) : shape_of(table, epi, g.M);
   const dim3 grid(static_cast<unsigned>(groups_of(s, epi == kEpiSwiglu ? g.n_out : g.N)),
                   static_cast<unsigned>((g.M + s.rows - 1) / s.rows));
   hipLaunchKernelGGL(s.fn, grid, dim3(s.threads), 0, stream, a);

@@ -54,7 +54,12 @@ __device__ __forceinline__ v4f32 mfma16(v4i32 a, v4i32 b, v4f32 c) {
 // OUT: the output element type; ACC: C += A B instead of C = A B.  Both are
 // compile-time, so the common store (f16, no accumulate) carries no branches
 // (256^3: 2.20 us; 2.49 with them chosen at run time).
-template <typename T, int KS, typename OUT, bool ACC>
+//
+// KN: B is the plain [K, N] operand, in any alignment.  The wave reads its 16
+// columns of every K row (32 bytes, two lanes a row), keeps them in LDS and
+// picks its fragments out of the words of neighbouring rows, which takes the
+// place of a pack launch before this one (256^3: 2.6 + 2.3 us in a HIP graph).
+template <typename T, int KS, typename OUT, bool ACC, bool KN>
 __global__ __launch_bounds__(64) void small_gemm_kernel(SmallArgs g) {
   const int lane = threadIdx.x;
   const int r = lane & 15, kq = lane >> 4;
@@ -64,13 +69,49 @@ __global__ __launch_bounds__(64) void small_gemm_kernel(SmallArgs g) {
   const uint8_t* b = g.B + static_cast<int64_t>(n < g.N ? n : g.N - 1) * g.ldb_bytes;
   v4i32 av[KS], bv[KS];
   const v4i32 zero = {0, 0, 0, 0};
+  if constexpr (KN) {
+    constexpr int kPitch = 36;  // bytes per K row in LDS: 16 columns and a word
+    __shared__ __attribute__((aligned(16))) uint8_t tile[KS * 32 * kPitch];
+    const int half = lane & 1;
+    // The last chunk of a row is its last 16 bytes, shifted down.
+    const int at = min(n0 + half * 8, g.N - 8), out = min(n0 + half * 8 - at, 8);
+    v4i32 raw[KS];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    const int k = s * 32 + kq * 8;
-    const bool in = k < g.K;
-    av[s] = *reinterpret_cast<const v4i32*>(a + (in ? k : 0) * 2);
-    bv[s] = *reinterpret_cast<const v4i32*>(b + (in ? k : 0) * 2);
-    if (!in) av[s] = bv[s] = zero;
+    for (int s = 0; s < KS; ++s) {
+      const int k = s * 32 + (lane >> 1);
+      typedef v4i32 any __attribute__((aligned(1)));
+      raw[s] = *reinterpret_cast<const any*>(g.B + (k < g.K ? k : g.K - 1) * g.ldb_bytes + at * 2);
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int k = s * 32 + kq * 8;
+      av[s] = *reinterpret_cast<const v4i32*>(a + (k < g.K ? k : 0) * 2);
+      if (k >= g.K) av[s] = zero;
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int k = s * 32 + (lane >> 1);
+      unsigned __int128 v = __builtin_bit_cast(unsigned __int128, raw[s]);
+      v = k < g.K && out < 8 ? v >> (out * 16) : 0;
+      const v4u32_t o = __builtin_bit_cast(v4u32_t, v);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        *reinterpret_cast<uint32_t*>(tile + k * kPitch + half * 16 + e * 4) = o[e];
+    }
+    // One wave: its LDS operations complete in order, and the compiler keeps
+    // them so.
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int s = 0; s < KS; ++s) bv[s] = kn_fragment<2>(tile, kPitch, s * 32 + kq * 8, r * 2);
+  } else {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int k = s * 32 + kq * 8;
+      const bool in = k < g.K;
+      av[s] = *reinterpret_cast<const v4i32*>(a + (in ? k : 0) * 2);
+      bv[s] = *reinterpret_cast<const v4i32*>(b + (in ? k : 0) * 2);
+      if (!in) av[s] = bv[s] = zero;
+    }
   }
   // Two independent chains; their sum is one more fp32 rounding per output.
   v4f32 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
@@ -93,27 +134,27 @@ __global__ __launch_bounds__(64) void small_gemm_kernel(SmallArgs g) {
   }
 }
 
-template <typename T, int KS>
+template <typename T, int KS, bool KN>
 void launch_ks(const SmallArgs& g, dim3 grid, hipStream_t s) {
   if (g.out_dtype == HXM_F32)
-    g.accumulate ? small_gemm_kernel<T, KS, float, true><<<grid, 64, 0, s>>>(g)
-                 : small_gemm_kernel<T, KS, float, false><<<grid, 64, 0, s>>>(g);
+    g.accumulate ? small_gemm_kernel<T, KS, float, true, KN><<<grid, 64, 0, s>>>(g)
+                 : small_gemm_kernel<T, KS, float, false, KN><<<grid, 64, 0, s>>>(g);
   else if (g.out_dtype == HXM_F16)
-    g.accumulate ? small_gemm_kernel<T, KS, _Float16, true><<<grid, 64, 0, s>>>(g)
-                 : small_gemm_kernel<T, KS, _Float16, false><<<grid, 64, 0, s>>>(g);
+    g.accumulate ? small_gemm_kernel<T, KS, _Float16, true, KN><<<grid, 64, 0, s>>>(g)
+                 : small_gemm_kernel<T, KS, _Float16, false, KN><<<grid, 64, 0, s>>>(g);
   else
-    g.accumulate ? small_gemm_kernel<T, KS, __bf16, true><<<grid, 64, 0, s>>>(g)
-                 : small_gemm_kernel<T, KS, __bf16, false><<<grid, 64, 0, s>>>(g);
+    g.accumulate ? small_gemm_kernel<T, KS, __bf16, true, KN><<<grid, 64, 0, s>>>(g)
+                 : small_gemm_kernel<T, KS, __bf16, false, KN><<<grid, 64, 0, s>>>(g);
 }
 
-template <typename T>
+template <typename T, bool KN>
 hxm_status launch_t(const SmallArgs& g, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((g.N + 15) / 16), static_cast<unsigned>((g.M + 15) / 16));
   const int ks = (g.K + 31) / 32;
-  if (ks <= 1) launch_ks<T, 1>(g, grid, s);
-  else if (ks <= 2) launch_ks<T, 2>(g, grid, s);
-  else if (ks <= 4) launch_ks<T, 4>(g, grid, s);
-  else launch_ks<T, 8>(g, grid, s);
+  if (ks <= 1) launch_ks<T, 1, KN>(g, grid, s);
+  else if (ks <= 2) launch_ks<T, 2, KN>(g, grid, s);
+  else if (ks <= 4) launch_ks<T, 4, KN>(g, grid, s);
+  else launch_ks<T, 8, KN>(g, grid, s);
   return check_launch("small gemm");
 }
 
@@ -133,8 +174,8 @@ bool small_gemm_fits(int64_t M, int64_t N, int64_t K, int32_t ab_dtype) {
 }
 
 hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const uint8_t* B,
-                             int64_t ldb_bytes, void* C, int64_t ldc, int64_t M, int64_t N,
-                             int64_t K, int32_t out_dtype, int32_t accumulate,
+                             int64_t ldb_bytes, bool kn, void* C, int64_t ldc, int64_t M,
+                             int64_t N, int64_t K, int32_t out_dtype, int32_t accumulate,
                              hipStream_t stream) {
   SmallArgs g;
   g.A = static_cast<const uint8_t*>(A);
@@ -148,7 +189,11 @@ hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const
   g.K = static_cast<int>(K);
   g.out_dtype = out_dtype;
   g.accumulate = accumulate;
-  return ab_dtype == HXM_BF16 ? launch_t<__bf16>(g, stream) : launch_t<_Float16>(g, stream);
+  if (kn)
+    return ab_dtype == HXM_BF16 ? launch_t<__bf16, true>(g, stream)
+                                : launch_t<_Float16, true>(g, stream);
+  return ab_dtype == HXM_BF16 ? launch_t<__bf16, false>(g, stream)
+                              : launch_t<_Float16, false>(g, stream);
 }
 
 }  // namespace hxm

@@ -568,7 +568,7 @@ hxm_status hxm_gemv_w8a16(const void* x, int64_t ldx, const int8_t* W, int64_t l
     a.N = g.N;
     a.K_bytes = g.K * 2;
     a.col_scale = static_cast<const float*>(w_scale);  // f16 values (kEpiGemv)
-    return launch_skinny(kSkinnyW8, kEpiGemv, a, s);
+    return launch_skinny(kSkinnyW8, kEpiGemv, a, false, s);
   }
   // Channel groups per workgroup at M > 4 (packed image): three share each
   // staged x chunk, which pays while a workgroup per 16 channels would more

@@ -87,9 +87,11 @@ hxm_gemm_config small_gemm_config();
 bool is_small_gemm_config(const hxm_gemm_config& c);
 bool small_gemm_fits(int64_t M, int64_t N, int64_t K, int32_t ab_dtype);
 hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const uint8_t* B,
-                             int64_t ldb_bytes, void* C, int64_t ldc, int64_t M, int64_t N,
-                             int64_t K, int32_t out_dtype, int32_t accumulate,
+                             int64_t ldb_bytes, bool kn, void* C, int64_t ldc, int64_t M,
+                             int64_t N, int64_t K, int32_t out_dtype, int32_t accumulate,
                              hipStream_t stream);
+// kn: B is the plain [K, N] operand, in any alignment, of rows of 16 bytes or more.
+inline bool small_takes_kn(int64_t N) { return N >= 8; }
 
 // Operand packs (pack.hip).  [K, N] (elements of eb = 1 or 2 bytes, row stride
 // ldb) -> the [N, K] image of row stride ldo; the same from f32 to fp16; and the

@@ -62,7 +62,12 @@ struct SkinnyArgs {
 // admit operands whose 256 rows lie within 2 GiB).
 constexpr uint32_t kSkOob = 0x40000000u;
 
-template <int KIND, int MR, int CB, int NW, int SL, int U, int EPI>
+// KN (f16, bf16 and int8): B is the plain [K, N] operand instead, in any
+// alignment.  A slab is then SL bytes of A's K as rows of 16 * CB channels, and
+// the words of neighbouring K rows are put together into fragments as they
+// leave LDS (kn_fragment), so the call needs no transposed copy of B: packing
+// one reads, writes and reads again what this reads once.
+template <int KIND, int MR, int CB, int NW, int SL, int U, int EPI, bool KN = false>
 __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
   constexpr bool W8 = KIND == kSkW8;
   constexpr int XL = W8 ? 2 : 1;       // A bytes per weight byte
@@ -77,7 +82,13 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
   constexpr int AN = (MR * AL + 63) / 64;                     // A loads per slab
   constexpr int kWRow = SL + 16, kARow = SL * XL + 16;
   constexpr int kARows = AN * 64 / AL;                        // staged A rows (>= MR)
-  constexpr int kSlab = CB * 16 * kWRow + kARows * kARow;
+  constexpr int EB = KIND == kSkF16 || KIND == kSkBF16 ? 2 : 1;
+  constexpr int kKnRows = SL / EB, kKnBytes = 16 * CB * EB;   // KN: slab rows, bytes of each
+  constexpr int kKnPitch = kKnBytes + 4, RL = kKnBytes / 16;  // lanes per row
+  static_assert(!KN || (!W8 && (EPI == kEpiFloat || EPI == kEpiI32 || EPI == kEpiDequant) &&
+                        (kKnPitch * kKnRows) % 16 == 0), "[K, N] operands");
+  constexpr int WL_N = KN ? kKnRows * RL / 64 : CB * WN;      // weight loads per slab
+  constexpr int kSlab = (KN ? kKnRows * kKnPitch : CB * 16 * kWRow) + kARows * kARow;
   using acc_t = typename std::conditional<KIND == kSkI8, v4i32, v4f32>::type;
   constexpr int MC = MT * CB <= 4 ? MT : (4 / CB > 0 ? 4 / CB : 1);  // row blocks per reduction round
   constexpr int TC = MC * CB;                                        // tiles per round
@@ -108,7 +119,8 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
       return (blk * CB + c) * 16;
     }
   };
-  __amdgpu_buffer_rsrc_t wr[CB];
+  __amdgpu_buffer_rsrc_t wr[KN ? 1 : CB];
+  if constexpr (!KN)
 #pragma unroll
   for (int c = 0; c < CB; ++c) {
     const int row0 = b_row0(c);
@@ -141,8 +153,13 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
     for (int c = 0; c < CB; ++c) acc[t][c] = acc_t{};
 
   struct Batch {
-    v4i32 w[U][CB][WN], a[U][AN];
+    v4i32 w[U][WL_N], a[U][AN];
   };
+  // KN: the lane's chunk of a row -- the row's last one is the last 16 bytes
+  // of B's row, shifted down -- and the K rows it takes.
+  const int kn_n = blk * (16 * CB) + (lane % RL) * (16 / EB);
+  const int kn_at = min(kn_n, g.N - 16 / EB), kn_out = min(kn_n - kn_at, 16 / EB);
+  const int kn_k = lane / RL, K = g.KB / EB;
   const int slabs = (g.KB + SL - 1) / SL;
   auto load = [&](Batch& q, int s0) {
 #pragma unroll
@@ -150,12 +167,22 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
       const int k0 = (s0 * U + u) * SL;
       const uint32_t wk = k0 + (k0 + wc < g.KB ? 0u : kSkOob);
       const uint32_t ak = k0 * XL + (k0 * XL + ac < g.KB * XL ? 0u : kSkOob);
+      if constexpr (KN) {
+        // Rows past K load row K - 1 (they are zeroed on the way to LDS).
 #pragma unroll
-      for (int c = 0; c < CB; ++c)  // nontemporal: the weights are streamed once
+        for (int t = 0; t < WL_N; ++t) {
+          const int k = min(k0 / EB + t * (64 / RL) + kn_k, K - 1);
+          typedef v4i32 any __attribute__((aligned(1)));
+          q.w[u][t] = *reinterpret_cast<const any*>(g.B + k * g.ldb_bytes + kn_at * EB);
+        }
+      } else {
 #pragma unroll
-        for (int t = 0; t < WN; ++t)
-          q.w[u][c][t] = __builtin_bit_cast(
-              v4i32, __builtin_amdgcn_raw_buffer_load_b128(wr[c], woff[t] + wk, 0, 2));
+        for (int c = 0; c < CB; ++c)  // nontemporal: the weights are streamed once
+#pragma unroll
+          for (int t = 0; t < WN; ++t)
+            q.w[u][c * WN + t] = __builtin_bit_cast(
+                v4i32, __builtin_amdgcn_raw_buffer_load_b128(wr[c], woff[t] + wk, 0, 2));
+      }
 #pragma unroll
       for (int t = 0; t < AN; ++t)
         q.a[u][t] = __builtin_bit_cast(
@@ -163,20 +190,38 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
     }
   };
   uint8_t* const area = lds + wave * (U * kSlab);
-  auto multiply = [&](const Batch& q) {
+  auto multiply = [&](const Batch& q, int s0) {
+    asm volatile("" ::: "memory");  // the previous slab's reads come first
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       uint8_t* const as = area + u * kSlab;
       uint8_t* const ws = as + kARows * kARow;
+      if constexpr (KN) {
 #pragma unroll
-      for (int c = 0; c < CB; ++c)
+        for (int t = 0; t < WL_N; ++t) {
+          const int row = t * (64 / RL) + kn_k;
+          const bool in = (s0 * U + u) * kKnRows + row < K;
+          unsigned __int128 v = __builtin_bit_cast(unsigned __int128, q.w[u][t]);
+          v = in && kn_out < 16 / EB ? v >> (kn_out * 8 * EB) : 0;
+          const v4u32_t o = __builtin_bit_cast(v4u32_t, v);
 #pragma unroll
-        for (int t = 0; t < WN; ++t)
-          *reinterpret_cast<v4i32*>(ws + (c * 16 + t * (64 / WL) + wr_) * kWRow + wc) = q.w[u][c][t];
+          for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint32_t*>(ws + row * kKnPitch + (lane % RL) * 16 + e * 4) = o[e];
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+#pragma unroll
+          for (int t = 0; t < WN; ++t)
+            *reinterpret_cast<v4i32*>(ws + (c * 16 + t * (64 / WL) + wr_) * kWRow + wc) =
+                q.w[u][c * WN + t];
+      }
 #pragma unroll
       for (int t = 0; t < AN; ++t)
         *reinterpret_cast<v4i32*>(as + (t * (64 / AL) + ar_) * kARow + ac) = q.a[u][t];
     }
+    // One wave's LDS operations complete in order; this keeps the compiler's.
+    asm volatile("" ::: "memory");
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint8_t* const as = area + u * kSlab;
@@ -192,7 +237,11 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
                 as + (MR < 16 ? r16 % kARows : t * 16 + r16) * kARow + ((j * 4 + kq) * XL + h) * 16);
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
-          const v4i32 w = *reinterpret_cast<const v4i32*>(ws + (c * 16 + r16) * kWRow + (j * 4 + kq) * 16);
+          v4i32 w;
+          if constexpr (KN)
+            w = kn_fragment<EB>(ws, kKnPitch, (j * 4 + kq) * (16 / EB), (c * 16 + r16) * EB);
+          else
+            w = *reinterpret_cast<const v4i32*>(ws + (c * 16 + r16) * kWRow + (j * 4 + kq) * 16);
           if constexpr (W8) {
             const v8f16 wa = i8x8_to_f16<b_offset_binary(EPI)>(static_cast<uint32_t>(w[0]),
                                                                static_cast<uint32_t>(w[1]));
@@ -230,9 +279,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(SkinnyArgs g) {
   load(q0, wave);
   for (int s = wave; s < end; s += 2 * NW) {
     load(q1, s + NW);
-    multiply(q0);
+    multiply(q0, s);
     load(q0, s + 2 * NW);
-    if (s + NW < end) multiply(q1);
+    if (s + NW < end) multiply(q1, s + NW);
   }
   __syncthreads();  // the sums reuse the staging areas
 

@@ -76,7 +76,8 @@ typedef enum hxm_dtype {
  *   HXM_B_KN: B is [K,N] row-major with leading dimension ldb >= N -- the
  *             plain linalg.matmul operand.  The library packs it per call
  *             into a library-owned workspace (the reference's per-launch
- *             hmx.pack_weight, HmxOps.td:229).
+ *             hmx.pack_weight, HmxOps.td:229); the kernels for few rows and
+ *             small outputs read it as it is.
  *   HXM_B_NK: B is already packed, [N,K] row-major (K contiguous), ldb >= K --
  *             the resident image produced once by hxm_prepack_weight (the
  *             reference's weight-resident path, WeightResidentPass.cpp:10-53,
@@ -171,8 +172,9 @@ typedef struct hxm_plan {
   int32_t threads;         /* threads per workgroup */
   int64_t tiles;           /* output tiles (workgroups per K slice) */
   int64_t lds_bytes;       /* LDS per workgroup */
-  int64_t workspace_bytes; /* library-owned device bytes the call uses (B pack,
-                              split-K planes) */
+  int64_t workspace_bytes; /* library-owned device bytes the call uses at most (B
+                              pack, split-K planes; the small-output kernel
+                              itself reads a [K,N] B of 8 columns or more) */
   int64_t m, n, k;         /* the shape planned */
 } hxm_plan;
 

@@ -179,3 +179,55 @@ def test_gemv_plain_weights(dev, M, N, K):
     ref = orc.f16_bits_to_f32(orc.gemv_w8a16(bits(x), W.numpy(), bits(s)))
     np.testing.assert_allclose(y.float().cpu().numpy(), ref, **TOL)
     assert (ybuf[:, N:] == 7).all() and (ybuf[M:] == 7).all()
+
+
+@pytest.mark.parametrize("M", [1, 5, 32, 33, 100])
+@pytest.mark.parametrize("N,K", [(16, 16), (33, 272), (100, 2064), (333, 144)])
+def test_int8_reads_kn_operands_as_they_are(dev, M, N, K):
+    """A [K, N] B without a transposed copy, from rows off any alignment."""
+    print(f"skinny int8 kn M={M} N={N} K={K}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    B = torch.randint(-127, 128, (K, N), generator=g, dtype=torch.int8)
+    _, Ad = padded(A, 111, dev)
+    ref = orc.gemm_i8(A.numpy(), B.numpy())
+    for cols in (0, 3):
+        _, Bd = padded(B, 111, dev, rows=0, cols=cols)
+        C = ops.gemm_i8(Ad, Bd, config=SKINNY)
+        assert ops.last_plan()["workspace_bytes"] == 0
+        assert np.array_equal(C.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("M", [1, 5, 32, 33, 100])
+@pytest.mark.parametrize("N,K", [(8, 8), (9, 136), (33, 1032), (333, 72)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_float_reads_kn_operands_as_they_are(dev, dt, M, N, K):
+    print(f"skinny kn {dt} M={M} N={N} K={K}", flush=True)
+    name = "f16" if dt == torch.float16 else "bf16"
+    g = torch.Generator().manual_seed(M + N + K)
+    A = (torch.rand(M, K, generator=g) * 2 - 1).to(dt)
+    B = (torch.rand(K, N, generator=g) * 2 - 1).to(dt)
+    _, Ad = padded(A, float("nan"), dev)
+    ref = orc.matmul(bits(A), bits(B), ab_dtype=name, c_dtype="f32")
+    for cols in (0, 3):
+        _, Bd = padded(B, float("nan"), dev, rows=0, cols=cols)
+        c = ops.matmul(Ad, Bd, out_dtype=torch.float32, config=SKINNY)
+        np.testing.assert_allclose(c.cpu().numpy(), ref, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 8, 8), (17, 9, 40), (33, 31, 72), (100, 70, 200),
+                                   (256, 256, 256), (1, 500, 128)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_small_output_kernel_reads_kn_operands_as_they_are(dev, dt, M, N, K):
+    """The small-output kernel on a plain [K, N] B off any alignment gives the
+    bits it gives on the [N, K] image."""
+    print(f"small kn {dt} M={M} N={N} K={K}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    A = (torch.rand(M, K, generator=g) * 2 - 1).to(dt).to(dev)
+    B = (torch.rand(K, N, generator=g) * 2 - 1).to(dt)
+    want = ops.matmul(A, B.t().contiguous().to(dev), b_layout="nk")
+    for cols in (0, 3):
+        _, Bd = padded(B, float("nan"), dev, rows=0, cols=cols)
+        got = ops.matmul(A, Bd)
+        assert ops.last_plan()["config"] == (16, 16, 32, 1, 1, 0, 1)
+        assert torch.equal(got, want)
