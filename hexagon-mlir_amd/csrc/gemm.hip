@@ -569,6 +569,11 @@ bool w8_kernel_has_swiglu(int i) { return part_fn(kW8Parts, i, 1) != nullptr; }
 bool w8_kernel_has_stream_k(int i) { return i == 0; }
 static gemm_fn w8_stream_k_fn(int e) { return kW8SkParts[e][e]; }
 
+// K splits of the W8A16 GEMMs (fp32 partial planes): the 128x128 tile, 2 to 16.
+bool w8_split_valid(int i, int32_t s) { return i == kW8PartEntry && s >= 2 && s <= 16; }
+// Partial plane rows: the B rows rounded up to whole 16-byte quads.
+static int64_t w8_plane_ld(int64_t N) { return (N + 3) / 4 * 4; }
+
 static const KernelEntry* find_w8_kernel(const hxm_gemm_config& c, bool swiglu) {
   for (int i = 0; i < kNumW8Kernels; ++i) {
     const hxm_gemm_config k = w8_kernel_config(i);
@@ -576,27 +581,67 @@ static const KernelEntry* find_w8_kernel(const hxm_gemm_config& c, bool swiglu) 
         (c.waves_m == 0 || c.waves_m == k.waves_m) &&
         (c.waves_n == 0 || c.waves_n == k.waves_n) &&
         (c.stages == 0 || c.stages == k.stages) &&
-        (c.split_k == 0 || c.split_k == 1 ||
+        (c.split_k == 0 || c.split_k == 1 || w8_split_valid(i, c.split_k) ||
          (c.split_k == HXM_STREAM_K && w8_kernel_has_stream_k(i))) &&
-        (!swiglu || w8_kernel_has_swiglu(i)))
+        (!swiglu || w8_kernel_has_swiglu(i) || w8_split_valid(i, c.split_k)))
       return &kW8Kernels[i];
   }
   return nullptr;
 }
 
-// The first table entry (largest tiles first) that still gives every CU a
-// workgroup, else the entry with the most tiles.
-hxm_gemm_config default_w8_config(int64_t M, int64_t N, bool swiglu) {
-  int best = -1;
-  int64_t best_tiles = -1;
+// The untuned W8A16 kernel: up to 32 rows the skinny one, which streams the
+// weights faster than any tile; above, the shortest of the modeled times (us)
+// over it, the compiled tiles and the K splits of the 128x128 tile.  A stage
+// costs a workgroup that has its CU to itself `stage` (the 128x128 tile, of
+// which two fit a CU, kStage2 for both), a call `base`, a split's planes one
+// write and one read.  Fitted to 118 calls (33 to 1024 rows, N 512 to 22016, K
+// 736 to 11008, HIP graph, one box), where its choice is 1.4% from the best of
+// all kernels in the geometric mean.  Skinny / best tile / split: down 4096 x
+// 11008, 57 rows 27.3 / 67.3 / 18.3, 256 rows 114 / 67 / 32.6; gate/up 2048 x
+// 4096, 128 rows 13.8 / 39.4 / 17.8; 11008 x 4096, 57 rows 38 / 40 / 31.
+// Without splits (`splits` false) the same choice among the rest.
+hxm_gemm_config default_w8_config(int epi, int64_t M, int64_t N, int64_t n_out, int64_t K,
+                                  bool splits) {
+  static constexpr struct { double base, stage; } kCost[kNumW8Kernels] = {
+      {7.0, 0.94}, {7.0, 0.96}, {5.5, 0.53}, {6.0, 0.58}, {4.3, 0.37}};
+  constexpr double kStage2 = 0.70, kSplitBase = 9.2, kPlaneBytesPerUs = 6.2e6;
+  constexpr int64_t kCus = 256;
+  const bool swiglu = epi == kEpiSwiglu;
+  const auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const bool skinny = skinny_fits(M, n_out, K);
+  if (skinny && M <= 32) return skinny_config();
+  hxm_gemm_config best = w8_kernel_config(0);
+  double best_us = 1e300;
+  const auto offer = [&](const hxm_gemm_config& c, double us) {
+    if (us < best_us) best = c, best_us = us;
+  };
+  const auto walk2 = [&](int64_t groups, int64_t stages) {
+    const int64_t rem = groups % (2 * kCus);
+    return static_cast<double>(stages) *
+           (groups / (2 * kCus) * kStage2 +
+            (rem == 0 ? 0.0 : rem <= kCus ? kCost[kW8PartEntry].stage : kStage2));
+  };
   for (int i = 0; i < kNumW8Kernels; ++i) {
-    if (swiglu && !w8_kernel_has_swiglu(i)) continue;
-    const hxm_gemm_config k = w8_kernel_config(i);
-    const int64_t tiles = ((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
-    if (tiles >= 256) return k;
-    if (tiles > best_tiles) best = i, best_tiles = tiles;
+    const hxm_gemm_config c = w8_kernel_config(i);
+    const int64_t tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn), stages = ceil_div(K, c.bk);
+    if (!swiglu || w8_kernel_has_swiglu(i))
+      offer(c, kCost[i].base + (i == kW8PartEntry
+                                    ? walk2(tiles, stages)
+                                    : static_cast<double>(ceil_div(tiles, kCus) * stages) *
+                                          kCost[i].stage));
+    if (i != kW8PartEntry || !splits) continue;
+    for (int32_t s = 2; w8_split_valid(i, s) && tiles * s <= 2 * kCus && stages >= 4 * s; ++s) {
+      hxm_gemm_config sc = c;
+      sc.split_k = s;
+      offer(sc, kSplitBase + walk2(tiles * s, ceil_div(stages, s)) +
+                    static_cast<double>(s * M) * w8_plane_ld(N) * 8 / kPlaneBytesPerUs);
+    }
   }
-  return w8_kernel_config(best);
+  if (skinny)
+    offer(skinny_config(), 1.0 + static_cast<double>(ceil_div(
+                                     skinny_groups(kSkinnyW8, epi, M, n_out), kCus)) *
+                                     (1.8 + static_cast<double>(K) / (swiglu ? 420 : 530)));
+  return best;
 }
 
 // The SwiGLU weight image: rows [128c, 128c+64) are gate channels
@@ -635,7 +680,8 @@ static int64_t stream_k_bytes(const KernelEntry& e, const StreamKLayout& sk) {
 // plan_gemm for the W8A16 GEMMs (f16 A, int8 [N, K] B): N is the B rows
 // (the SwiGLU image's), n_out the output columns.
 hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out, int64_t K,
-                        const hxm_gemm_config* cfg, hxm_plan* p, const KernelEntry** entry) {
+                        const hxm_gemm_config* cfg, bool splits, hxm_plan* p,
+                        const KernelEntry** entry) {
   *p = hxm_plan{};
   p->op = op;
   p->m = M, p->n = n_out, p->k = K;
@@ -650,7 +696,7 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
   } else if (lookup_tuned(op, M, sw ? n_out : N, K, &c)) {
     p->source = HXM_SOURCE_TUNED;
   } else {
-    c = skinny_default(kSkinnyW8, epi, M, n_out, K) ? skinny_config() : default_w8_config(M, N, sw);
+    c = default_w8_config(epi, M, N, n_out, K, splits);
     p->source = HXM_SOURCE_DEFAULT;
   }
   p->config = c;
@@ -681,7 +727,13 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
     p->tiles = ((M + e->cfg.bm - 1) / e->cfg.bm) * ((N + e->cfg.bn - 1) / e->cfg.bn);
     p->lds_bytes = kernel_lds_bytes(*e, true, false);
     int64_t groups = p->tiles, sk_tiles = 0;
-    if (c.split_k == HXM_STREAM_K) {
+    bool planes_fit = true;
+    if (w8_split_valid(static_cast<int>(e - kW8Kernels), c.split_k)) {
+      p->k_slices = k_slices(K * 2, e->cfg.bk, c.split_k);
+      p->config.split_k = c.split_k;
+      planes_fit = split_planes_fit(p->k_slices, M, w8_plane_ld(N), kSplitKPlaneBytesMax);
+      if (planes_fit) p->workspace_bytes = p->k_slices * M * w8_plane_ld(N) * 4;
+    } else if (c.split_k == HXM_STREAM_K) {
       // Stream-K when the tiles leave a partial round; whole rounds run as
       // split_k = 1.  The plan records the mode, the partial-tile slots (as
       // k_slices: the most workgroups one tile is cut over) and the buffer.
@@ -695,7 +747,11 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
         sk_tiles = sk.tiles;
       }
     }
-    if (p->workspace_bytes > kSplitKPlaneBytesMax) {
+    if (!planes_fit) {
+      snprintf(why, sizeof(why), "split_k=%d needs %d fp32 partial planes above the %lld-byte limit",
+               c.split_k, p->k_slices, (long long)kSplitKPlaneBytesMax);
+      st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_WORKSPACE_BUDGET, why);
+    } else if (p->workspace_bytes > kSplitKPlaneBytesMax) {
       snprintf(why, sizeof(why),
                "stream-K needs %lld bytes of fp32 partial tiles, above the %lld-byte limit",
                (long long)p->workspace_bytes, (long long)kSplitKPlaneBytesMax);
@@ -704,7 +760,8 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
       snprintf(why, sizeof(why), "stream-K with %lld partial-round tiles needs more than %lld "
                "arrival counters", (long long)sk_tiles, (long long)(kStreamKCounterBytes / 4));
       st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_WORKSPACE_BUDGET, why);
-    } else if (!grid_fits(groups, e->threads)) {
+    } else if (!grid_fits(groups, e->threads,
+                          p->config.split_k == HXM_STREAM_K ? 1 : p->k_slices)) {
       snprintf(why, sizeof(why), "%lld workgroups of %d threads exceed the launch limit",
                (long long)groups, e->threads);
       st = refuse(p, HXM_UNSUPPORTED_SHAPE, HXM_REASON_TILE_ALIGNMENT, why);
@@ -727,10 +784,20 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
   const bool sw = epi == kEpiSwiglu;
   const KernelEntry* e = nullptr;
   hxm_plan plan;
-  hxm_status st = plan_gemm_w8(op, epi, M, N, n_out, K, cfg, &plan, &e);
+  hxm_status st = plan_gemm_w8(op, epi, M, N, n_out, K, cfg, true, &plan, &e);
   if (st != HXM_OK) return st;
   if ((st = require_device(nullptr)) != HXM_OK) return st;
   if (M == 0 || N == 0) return ok();
+  void* planes = nullptr;
+  if (e && w8_split_valid(static_cast<int>(e - kW8Kernels), plan.config.split_k)) {
+    // An untuned call works on any stream at any time: where the planes cannot
+    // be had (a capture that would have to grow them, no memory) it runs the
+    // best kernel without them.
+    st = stream_workspace(stream, static_cast<size_t>(plan.workspace_bytes), &planes, kWsSplitK);
+    if (st != HXM_OK && plan.source == HXM_SOURCE_DEFAULT)
+      st = plan_gemm_w8(op, epi, M, N, n_out, K, cfg, false, &plan, &e);
+    if (st != HXM_OK) return st;
+  }
   GemmArgs g;
   g.A = static_cast<const uint8_t*>(x);
   g.B = reinterpret_cast<const uint8_t*>(W);
@@ -781,6 +848,30 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
     g.sk_count = static_cast<uint32_t*>(ws);
     g.sk_part = reinterpret_cast<float*>(static_cast<char*>(ws) + kStreamKCounterBytes);
     groups = sk.dp + sk.groups;
+  }
+  if (planes) {
+    const int S = plan.k_slices;
+    const int64_t ldp = w8_plane_ld(N), bkb = e->cfg.bk;
+    GemmArgs q = g;
+    q.C = planes;
+    q.ldc = ldp;
+    q.out_dtype = HXM_F32;
+    q.vec_store = q.vec8_store = 1;
+    q.residual = nullptr;
+    q.col_scale = nullptr;
+    q.split = S;
+    q.kslice_bytes =
+        static_cast<int>((K * 2 + bkb - 1) / bkb + plan.config.split_k - 1) / plan.config.split_k *
+        static_cast<int>(bkb);
+    q.plane_elems = M * ldp;
+    hipLaunchKernelGGL(kW8PartFns[sw ? 1 : 0],
+                       dim3(static_cast<unsigned>(plan.tiles), static_cast<unsigned>(S)),
+                       dim3(e->threads), 0, stream, q);
+    if ((st = check_launch("w8a16 split gemm")) != HXM_OK) return st;
+    if ((st = launch_w8_reduce(epi, g, static_cast<const float*>(planes), S, ldp, stream)) !=
+        HXM_OK)
+      return st;
+    return ok();
   }
   const int fe = sw ? 1 : epi == kEpiW8Res ? 2 : 0;
   hipLaunchKernelGGL(plan.config.split_k == HXM_STREAM_K ? w8_stream_k_fn(fe)

@@ -62,21 +62,25 @@ enum Epilogue {
   kEpiW8 = 3,       // f16 A x int8 B: f16(acc * cs[n])
   kEpiSwiglu = 4,   // f16 A x int8 gate/up image: f16(silu(g * sg) * (u * su))
   kEpiW8Res = 5,    // f16 A x int8 B: f16((acc * cs[n]) + r[m, n]), fp32 sum
-  kEpiGemv = 6      // f16 A x int8 B: f16(acc * cs16[n]), f16 scales (skinny only)
+  kEpiGemv = 6,     // f16 A x int8 B: f16(acc * cs16[n]), f16 scales (skinny only)
+  kEpiW8Part = 7,   // f16 A x int8 B: the fp32 accumulators (a K split's plane)
+  kEpiSwPart = 8    // the same from the gate/up image
 };
 
 // The int8-weight epilogues take B as int8 [N, K] converted to f16 in
 // registers (the W8A16 GEMM of the SwiGLU FFN).
 constexpr bool b_is_int8(int epi) {
-  return epi == kEpiW8 || epi == kEpiSwiglu || epi == kEpiW8Res || epi == kEpiGemv;
+  return epi == kEpiW8 || epi == kEpiSwiglu || epi == kEpiW8Res || epi == kEpiGemv ||
+         epi == kEpiW8Part || epi == kEpiSwPart;
 }
+constexpr bool is_w8_part(int epi) { return epi == kEpiW8Part || epi == kEpiSwPart; }
 // The SwiGLU image (built by this library, never by the caller) stores each
 // weight in offset binary, byte = w + 128 (w ^ 0x80 as a bit pattern): that
 // byte is the low byte of the f16 1024 + byte = 1152 + w directly, so the
 // conversion skips the sign flip the two's-complement B of kEpiW8 /
 // kEpiW8Res needs (eight VALU operations per 8 weights instead of ten;
 // gate/up of the FFN block at 2048x4096x11008 ran 302.5 -> 297.1 us).
-constexpr bool b_offset_binary(int epi) { return epi == kEpiSwiglu; }
+constexpr bool b_offset_binary(int epi) { return epi == kEpiSwiglu || epi == kEpiSwPart; }
 constexpr int32_t kOpW8 = HXM_OP_W8A16, kOpSwiglu = HXM_OP_W8A16_SWIGLU;  // tuning-cache keys
 
 // 16-byte f16 output store.  The int8-weight epilogues write activations
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
   static_assert(!SK || BQ, "stream-K is compiled for the int8-weight kernels");
   // Epilogue scales in LDS: rows [0, QR*64), columns [QR*64, (QR+QC)*64) floats.
   constexpr int QR = EPI == kEpiDequant ? (BM + 63) / 64 : 0;
-  constexpr int QC = EPI == kEpiDequant || BQ ? (BN + 63) / 64 : 0;
+  constexpr int QC = EPI == kEpiDequant || (BQ && !is_w8_part(EPI)) ? (BN + 63) / 64 : 0;
 
   // One __shared__ object per stage (see the header comment).
   __shared__ __attribute__((aligned(1024))) uint8_t s0[SB];
@@ -1028,7 +1032,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
       continue;
     }
   }
-  if constexpr (EPI == kEpiI32 || EPI == kEpiFloat) {
+  if constexpr (EPI == kEpiI32 || EPI == kEpiFloat || is_w8_part(EPI)) {
     // Plain overwrite (full tiles, or edge tiles with N % 4 == 0):
     // 4-element runs, one row address per block, a per-run check only on
     // edge tiles.
@@ -1303,6 +1307,15 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
 }
 
 typedef void (*gemm_fn)(GemmArgs);
+
+// The W8A16 K split (gemm_w8part.hip): kernels of entry kW8PartEntry of
+// HXM_W8_CONFIG_LIST that write fp32 partial planes ({kEpiW8Part, kEpiSwPart}),
+// and the pass that adds the S planes ([S][M][ldp], plane order) and runs the
+// epilogue of g.
+constexpr int kW8PartEntry = 4;
+extern const gemm_fn kW8PartFns[2];
+hxm_status launch_w8_reduce(int epi, const GemmArgs& g, const float* planes, int S, int64_t ldp,
+                            hipStream_t stream);
 
 // The skinny matmul (gemm_skinny.hip): fills a plan's config, threads, tiles
 // and LDS; launches (g as for the tile kernels; n_out the output columns).

@@ -103,18 +103,18 @@ bool skinny_fits(int64_t M, int64_t N, int64_t K) {
 // best tile us, HIP graph, one box): 4096 x 4096, 64: 13.2 / 14.4 (256
 // workgroups); 1024 x 4096, 256: 11.2 / 14.0 (256); 2048 x 4096, 192: 19.3 /
 // 14.4 (384); below 2 KiB of K the tiles' fixed time is the shorter one (4096 x
-// 512, 64: 4.4 / 4.1). int8 alike. f16 x int8 against its 128-row tiles,
-// down projection 4096 x 2048: 64 rows 7.1 / 16.1 (256), 128 12.8 / 16.2 (512),
-// 192 17.9 / 16.4 (768); gate/up 2048 x 4096: 256 rows 23.9 / 40.7 (512),
-// 11008 x 4096: 64 rows 42.1 / 41.2 (688), 96 70.8 / 41.8 (1376).
+// 512, 64: 4.4 / 4.1). int8 alike; the f16 x int8 calls are default_w8_config's.
 bool skinny_default(int32_t table, int epi, int64_t M, int64_t n_out, int64_t K) {
   if (!skinny_fits(M, n_out, K)) return false;
-  const int64_t kb = table == kSkinnyW8 ? K : K * dtype_bytes(table);
-  if (M <= 32) return table == kSkinnyW8 || kb >= 256;
+  const int64_t kb = K * dtype_bytes(table);
+  if (M <= 32) return kb >= 256;
+  return kb >= 2048 && skinny_groups(table, epi, M, n_out) <= 256;
+}
+
+// Workgroups of a call.
+int64_t skinny_groups(int32_t table, int epi, int64_t M, int64_t n_out) {
   const SkinnyShape s = shape_of(table, epi, M);
-  const int64_t groups = groups_of(s, n_out) * ((M + s.rows - 1) / s.rows);
-  if (table == kSkinnyW8) return groups <= (epi == kEpiSwiglu ? 700 : 512);
-  return kb >= 2048 && groups <= 256;
+  return groups_of(s, n_out) * ((M + s.rows - 1) / s.rows);
 }
 
 void skinny_plan(int32_t table, int epi, int64_t M, int64_t n_out, bool kn, hxm_plan* p) {

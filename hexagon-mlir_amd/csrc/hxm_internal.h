@@ -60,6 +60,9 @@ constexpr int kWsMain = 0, kWsSplitK = 1, kWsStreamK = 2;
 constexpr int64_t kSplitKPlaneBytesMax = int64_t(256) << 20;
 // Slot 2 holds the W8A16 stream-K partial tiles and arrival counters.
 // *grown (when given) says whether the buffer was (re)allocated by this call.
+// True while `stream` captures a graph, or when that cannot be read (the null
+// stream during another stream's global-mode capture).
+bool stream_capturing(hipStream_t stream);
 hxm_status stream_workspace(hipStream_t stream, size_t bytes, void** out, int slot = kWsMain,
                             bool* grown = nullptr);
 // CUs of the current device (cached per device; 0 when it cannot be read).
@@ -112,6 +115,7 @@ hxm_status pack_f32_operands(const float* A, int64_t lda, _Float16* ai, int64_t 
 constexpr int64_t kSkinnyRowsMax = 256;
 constexpr int32_t kSkinnyW8 = 0;
 bool skinny_default(int32_t table, int epi, int64_t M, int64_t n_out, int64_t K);
+int64_t skinny_groups(int32_t table, int epi, int64_t M, int64_t n_out);
 hxm_gemm_config skinny_config();
 bool is_skinny_config(const hxm_gemm_config& c);
 bool skinny_fits(int64_t M, int64_t N, int64_t K);

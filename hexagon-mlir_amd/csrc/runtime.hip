@@ -17,6 +17,8 @@ thread_local std::string g_last_error;
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
+  bool captured = false;       // ptr has been handed to a capturing stream
+  std::vector<void*> retired;  // earlier buffers that graphs hold
 };
 std::mutex g_ws_mu;
 // One buffer per (device, stream handle, slot).  The handle is compared as a
@@ -96,12 +98,20 @@ int device_cu_count() {
   return cus[dev];
 }
 
+bool stream_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamIsCapturing(stream, &cap);
+  if (e != hipSuccess) (void)hipGetLastError();  // clear the sticky query error
+  return e != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
+
 hxm_status stream_workspace(hipStream_t stream, size_t bytes, void** out, int slot, bool* grown) {
   int dev = 0;
   if (grown) *grown = false;
   HXM_HIP_TRY(hipGetDevice(&dev));
   if (slot != kWsMain && slot != kWsSplitK && slot != kWsStreamK)
     return fail(HXM_INVALID_ARG, "invalid-argument: workspace slot %d", slot);
+  const bool capturing = stream_capturing(stream);
   const WsKey key(dev, reinterpret_cast<uintptr_t>(stream), slot);
   std::lock_guard<std::mutex> lk(g_ws_mu);
   Workspace& w = g_ws[key];
@@ -111,25 +121,31 @@ hxm_status stream_workspace(hipStream_t stream, size_t bytes, void** out, int sl
     // that fails counts as a capture: the null stream, for one, reports an
     // implicit-capture error while another stream captures in global mode,
     // and a synchronisation or hipMalloc then would invalidate that capture.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const hipError_t qe = hipStreamIsCapturing(stream, &cap);
-    if (qe != hipSuccess) (void)hipGetLastError();  // clear the sticky query error
-    if (qe != hipSuccess || cap != hipStreamCaptureStatusNone)
+    if (capturing)
       return fail(HXM_UNSUPPORTED_SHAPE,
                   "workspace-budget: the stream is capturing a graph (or its capture state "
-                  "cannot be read: %s) and its workspace must grow from %zu to %zu bytes; "
+                  "cannot be read) and its workspace must grow from %zu to %zu bytes; "
                   "make one call of this shape on the stream before capturing (the workspace "
                   "is kept), or use hxm_gemm_i8_noalloc",
-                  qe == hipSuccess ? "capturing" : hipGetErrorString(qe), w.bytes, bytes);
-    if (w.ptr) {
+                  w.bytes, bytes);
+    size_t grow = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+    if (w.ptr && w.captured) {
+      // A graph holds the old buffer: it stays until hxm_release_cache().
+      // Doubling bounds what such buffers add up to by the newest one's size.
+      w.retired.push_back(w.ptr);
+      grow = std::max(grow, 2 * w.bytes);
+      w.ptr = nullptr;
+      w.bytes = 0;
+      w.captured = false;
+    } else if (w.ptr) {
       // The old buffer may still be read by work queued on this stream.
       HXM_HIP_TRY(hipStreamSynchronize(stream));
       HXM_HIP_TRY(hipFree(w.ptr));
       w.ptr = nullptr;
       w.bytes = 0;
     }
-    size_t grow = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
     if (hipMalloc(&w.ptr, grow) != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next launch
       w.ptr = nullptr;
       return fail(HXM_OUT_OF_MEMORY, "out-of-memory: workspace of %zu bytes",
                   grow);
@@ -137,6 +153,7 @@ hxm_status stream_workspace(hipStream_t stream, size_t bytes, void** out, int sl
     w.bytes = grow;
     if (grown) *grown = true;
   }
+  w.captured = w.captured || capturing;
   *out = w.ptr;
   return HXM_OK;
 }
@@ -184,6 +201,10 @@ hxm_status hxm_release_cache(void) {
   std::lock_guard<std::mutex> lk(hxm::g_ws_mu);
   for (auto it = hxm::g_ws.begin(); it != hxm::g_ws.end();) {
     if (std::get<0>(it->first) == dev) {
+      while (!it->second.retired.empty()) {
+        HXM_HIP_TRY(hipFree(it->second.retired.back()));
+        it->second.retired.pop_back();
+      }
       if (it->second.ptr) HXM_HIP_TRY(hipFree(it->second.ptr));
       it = hxm::g_ws.erase(it);
     } else {

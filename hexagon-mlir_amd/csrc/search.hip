@@ -40,7 +40,9 @@ int num_w8_kernels();
 hxm_gemm_config w8_kernel_config(int i);
 bool w8_kernel_has_swiglu(int i);
 bool w8_kernel_has_stream_k(int i);
-hxm_gemm_config default_w8_config(int64_t M, int64_t N, bool swiglu);
+bool w8_split_valid(int i, int32_t s);
+hxm_gemm_config default_w8_config(int epi, int64_t M, int64_t N, int64_t n_out, int64_t K,
+                                  bool splits);
 hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const int8_t* W,
                        int64_t ldw, const float* scale, void* C, int64_t ldc, int64_t M,
                        int64_t N, int64_t K, int64_t n_out, const hxm_gemm_config* cfg,
@@ -196,10 +198,14 @@ bool config_compiled(int32_t op, const hxm_gemm_config& c) {
     for (int i = 0; i < num_kernels(); ++i)
       if (same_config(kernel_config(i, op), base)) return true;
   } else if (op == HXM_OP_W8A16 || op == HXM_OP_W8A16_SWIGLU) {
-    for (int i = 0; i < num_w8_kernels(); ++i)
-      if (same_config(w8_kernel_config(i), c) &&
-          (op == HXM_OP_W8A16 || w8_kernel_has_swiglu(i)))
+    for (int i = 0; i < num_w8_kernels(); ++i) {
+      hxm_gemm_config base = c;
+      const bool split = w8_split_valid(i, c.split_k);  // a launch parameter
+      if (split) base.split_k = 1;
+      if (same_config(w8_kernel_config(i), base) &&
+          (op == HXM_OP_W8A16 || w8_kernel_has_swiglu(i) || split))
         return true;
+    }
   }
   return false;
 }
@@ -404,12 +410,12 @@ hxm_status tune_core(const TuneSpec& sp, int32_t reps, hxm_gemm_config* best, ch
     if (have_ref) {
       HXM_HIP_TRY(hipMemsetAsync(bad, 0, sizeof(unsigned), s));
       // The direct-load small-output kernel, the skinny kernel (partial sums
-      // of its waves) and the stream-K tiles (fp32 partial tiles added across
-      // workgroups) sum in another order than the staged one-workgroup tiles:
-      // checked within the float tolerance.
+      // of its waves) and the float K splits and stream-K tiles (fp32 partial
+      // sums added across workgroups) sum in another order than the staged
+      // one-workgroup tiles: checked within the float tolerance.
       if (is_small_gemm_config(cands[i]) != is_small_gemm_config(control) ||
           is_skinny_config(cands[i]) != is_skinny_config(control) ||
-          (cands[i].split_k == HXM_STREAM_K) != (control.split_k == HXM_STREAM_K))
+          (op != HXM_I8 && cands[i].split_k != control.split_k))
         count_far_kernel<<<1024, 256, 0, s>>>(static_cast<const uint32_t*>(C),
                                               (ldc * out_eb) / 4, ref, M, row_words,
                                               op == HXM_BF16, bad);
@@ -938,14 +944,23 @@ hxm_status hxm_tune_w8a16(int32_t op, const void* x, int64_t ldx, const int8_t* 
   TuneSpec sp;
   sp.op = op;
   sp.M = M, sp.N = N, sp.K = K;
+  sp.control = default_w8_config(epi, M, rows, N, K, true);
+  std::vector<hxm_gemm_config> splits;
   // Every compiled tile, and its stream-K form where its tiles leave a
   // partial round on this device.
   const int cus = device_cu_count();
   for (int i = 0; i < num_w8_kernels(); ++i) {
-    if (sw && !w8_kernel_has_swiglu(i)) continue;
     hxm_gemm_config c = w8_kernel_config(i);
-    sp.cands.push_back(c);
     const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((rows + c.bn - 1) / c.bn);
+    // K splits (powers of two, and the untuned call's own).
+    for (int32_t s = 2; w8_split_valid(i, s) && tiles * s <= 2 * cus && (K + c.bk - 1) / c.bk >= s;
+         ++s) {
+      hxm_gemm_config sc = c;
+      sc.split_k = s;
+      if ((s & (s - 1)) == 0 || same_config(sc, sp.control)) splits.push_back(sc);
+    }
+    if (sw && !w8_kernel_has_swiglu(i)) continue;
+    sp.cands.push_back(c);
     StreamKLayout sk;
     if (w8_kernel_has_stream_k(i) && stream_k_layout(tiles, (K + c.bk - 1) / c.bk, cus, &sk)) {
       c.split_k = HXM_STREAM_K;
@@ -953,10 +968,10 @@ hxm_status hxm_tune_w8a16(int32_t op, const void* x, int64_t ldx, const int8_t* 
     }
   }
   sort_configs(&sp.cands);
-  sp.control = default_w8_config(M, rows, sw);
   sp.canary = sp.cands.front();  // the smallest compiled tile on a 32-row slice
+  sp.cands.insert(sp.cands.end(), splits.begin(), splits.end());
+  sort_configs(&sp.cands);
   if (skinny_fits(M, N, K)) sp.cands.insert(sp.cands.begin(), skinny_config());
-  if (skinny_default(kSkinnyW8, epi, M, N, K)) sp.control = skinny_config();
   sp.cm = std::min<int64_t>(32, M), sp.cn = std::min<int64_t>(sw ? 64 : 32, N);
   sp.ck = std::min<int64_t>(K, 32);
   sp.run = [=](const hxm_gemm_config& c, int64_t m, int64_t n, int64_t k) {

@@ -23,7 +23,8 @@
  *     allocate or synchronise and may not.  A compute entry that uses the
  *     per-stream workspace (f32 operands, a [K,N] B, a K split) needs it
  *     already large enough: one call of the shape on the stream before the
- *     capture grows it (it is kept until hxm_release_cache).
+ *     capture grows it (it is kept until hxm_release_cache, also past a later
+ *     growth once a graph has captured it).
  *   - numerics: fp16/bf16 products accumulate in fp32 and are rounded once
  *     to the output dtype; int8 products accumulate exactly in int32.
  *   - host threads: entries may run at the same time on several host
@@ -97,8 +98,14 @@ typedef struct hxm_gemm_config {
                                S * M * N * 4 bytes, live in a library-owned
                                per-stream buffer kept until hxm_release_cache();
                                above 256 MiB the call is refused
-                               ("workspace-budget").  HXM_STREAM_K: the W8A16
-                               GEMMs' stream-K mode (below) */
+                               ("workspace-budget").  W8A16 GEMMs, 128x128 tile:
+                               2 to 16, fp32 planes summed in order, also the
+                               default of calls with few tiles and a long K
+                               (where the planes cannot be had, as in a capture
+                               that would have to grow them, an untuned call runs
+                               unsplit).
+                               HXM_STREAM_K: the W8A16 GEMMs' stream-K mode
+                               (below) */
 } hxm_gemm_config;
 
 /* split_k of a W8A16 GEMM config (hxm_gemm_w8a16, _swiglu, _residual): when

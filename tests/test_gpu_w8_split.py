@@ -1,0 +1,104 @@
+"""The K split of the W8A16 GEMMs (csrc/gemm_w8part.hip) against the CPU oracle:
+one slice to more slices than stages fill, rows and channels that end inside a
+tile and a four-column run, output rows off every alignment; the untuned choice
+of it; and its planes under graph capture."""
+import numpy as np
+import pytest
+import torch
+
+import hxm.ops as ops
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+# fp32 sums of f16 x int8 products in any order, one f16 rounding: the
+# tolerance the W8A16 entries state.
+TOL = dict(rtol=1e-2, atol=1e-3)
+
+
+def bits(t):
+    return t.contiguous().view(torch.int16).cpu().numpy().view(np.uint16)
+
+
+def operands(M, N, K, n_weights=1):
+    g = torch.Generator().manual_seed(M * 1000 + N + K)
+    x = torch.randn(M, K, generator=g).half()
+    W = [torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8) for _ in range(n_weights)]
+    s = [torch.rand(N, generator=g) * 0.004 + 0.001 for _ in range(n_weights)]
+    return g, x, W, s
+
+
+def padded(M, N, dev, pad):
+    buf = torch.full((M + 1, N + pad), 7.0, dtype=torch.float16, device=dev)
+    return buf, buf[:M, :N]
+
+
+def untouched(buf, M, N):
+    return bool((buf[:, N:] == 7).all() and (buf[M:] == 7).all())
+
+
+@pytest.mark.parametrize("M,N,K,S", [(1, 1, 16, 2), (57, 333, 656, 2), (128, 128, 1024, 16),
+                                     (129, 130, 2064, 5), (57, 258, 1040, 16), (300, 515, 720, 3)])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_against_oracle(dev, M, N, K, S, pad):
+    print(f"w8 split M={M} N={N} K={K} S={S} pad={pad}", flush=True)
+    cfg = (128, 128, 64, 2, 2, 3, S)
+    g, x, (W,), (s,) = operands(M, N, K)
+    r = (4 * torch.randn(M, N, generator=g)).half()
+    buf, y = padded(M, N, dev, pad)
+    ops.gemm_w8a16(x.to(dev), W.to(dev), s.to(dev), out=y, config=cfg)
+    assert ops.last_plan()["config"] == cfg
+    ref = orc.f16_bits_to_f32(orc.gemm_w8a16(bits(x), W.numpy(), s.numpy()))
+    np.testing.assert_allclose(y.float().cpu().numpy(), ref, **TOL)
+    assert untouched(buf, M, N)
+    buf, z = padded(M, N, dev, pad)                  # in place: out is the residual
+    z.copy_(r)
+    ops.gemm_w8a16(x.to(dev), W.to(dev), s.to(dev), out=z, residual=z, config=cfg)
+    ref = orc.f16_bits_to_f32(orc.gemm_w8a16_residual(bits(x), W.numpy(), s.numpy(), bits(r)))
+    np.testing.assert_allclose(z.float().cpu().numpy(), ref, **TOL)
+    assert untouched(buf, M, N)
+
+    _, x, (Wg, Wu), (sg, su) = operands(M, N, K, 2)
+    Wgu, sgu = ops.swiglu_pack(Wg.to(dev), Wu.to(dev), sg.to(dev), su.to(dev))
+    buf, h = padded(M, N, dev, pad)
+    ops.gemm_w8a16_swiglu(x.to(dev), Wgu, sgu, N, out=h, config=cfg)
+    ref = orc.f16_bits_to_f32(orc.swiglu_gateup(bits(x), Wg.numpy(), Wu.numpy(), sg.numpy(),
+                                                su.numpy()))
+    np.testing.assert_allclose(h.float().cpu().numpy(), ref, **TOL)
+    assert untouched(buf, M, N)
+
+
+def test_untuned_choice_and_capture(dev):
+    """57 rows of a long K are split when untuned.  A capture on a stream that
+    has the planes replays the eager call's bits, also after the planes have
+    grown; on a stream without them it runs unsplit instead of being refused."""
+    g, x, (W,), (s,) = operands(57, 1024, 8192)
+    x, W, s = x.to(dev), W.to(dev), s.to(dev)
+    y = torch.empty(57, 1024, dtype=torch.float16, device=dev)
+    warm, fresh = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(warm):
+        ops.gemm_w8a16(x, W, s, out=y)
+    plan = ops.last_plan()
+    assert plan["config"][6] > 1 and plan["workspace_bytes"] > 0
+    torch.cuda.synchronize()
+    want = y.clone()
+    graphs = []
+    for st, split in ((warm, True), (fresh, False)):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            ops.gemm_w8a16(x, W, s, out=y)
+        assert (ops.last_plan()["config"][6] > 1) == split
+        graphs.append(graph)
+    big = torch.randn(512, 8192, device=dev).half()
+    with torch.cuda.stream(warm):                    # grows that stream's planes
+        ops.gemm_w8a16(big, W, s, config=(128, 128, 64, 2, 2, 3, 16))
+    for rep in range(3):
+        for graph, exact in zip(graphs, (True, False)):
+            y.fill_(-7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            if exact:
+                assert torch.equal(y, want), rep
+            else:
+                torch.testing.assert_close(y, want, rtol=1e-2, atol=1e-3)
