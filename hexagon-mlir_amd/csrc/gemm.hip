@@ -569,8 +569,10 @@ bool w8_kernel_has_swiglu(int i) { return part_fn(kW8Parts, i, 1) != nullptr; }
 bool w8_kernel_has_stream_k(int i) { return i == 0; }
 static gemm_fn w8_stream_k_fn(int e) { return kW8SkParts[e][e]; }
 
-// K splits of the W8A16 GEMMs (fp32 partial planes): the 128x128 tile, 2 to 16.
-bool w8_split_valid(int i, int32_t s) { return i == kW8PartEntry && s >= 2 && s <= 16; }
+// K splits of the W8A16 GEMMs (fp32 partial planes), 2 to 16 slices.
+bool w8_split_valid(int i, int32_t s) {
+  return i >= kW8PartEntry && i < kW8PartEntry + kW8PartEntries && s >= 2 && s <= 16;
+}
 // Partial plane rows: the B rows rounded up to whole 16-byte quads.
 static int64_t w8_plane_ld(int64_t N) { return (N + 3) / 4 * 4; }
 
@@ -591,20 +593,21 @@ static const KernelEntry* find_w8_kernel(const hxm_gemm_config& c, bool swiglu) 
 
 // The untuned W8A16 kernel: up to 32 rows the skinny one, which streams the
 // weights faster than any tile; above, the shortest of the modeled times (us)
-// over it, the compiled tiles and the K splits of the 128x128 tile.  A stage
-// costs a workgroup that has its CU to itself `stage` (the 128x128 tile, of
-// which two fit a CU, kStage2 for both), a call `base`, a split's planes one
-// write and one read.  Fitted to 118 calls (33 to 1024 rows, N 512 to 22016, K
+// over it, the compiled tiles and the K splits of the 128x128 tile (the 64x128
+// one in its place up to 64 rows).  A stage costs a workgroup that has its CU to
+// itself `stage` (those two, of which two fit a CU, `stage2` for both), a call
+// `base`, a split's planes one write and one read.  Fitted to 118 calls (33 to 1024 rows, N 512 to 22016, K
 // 736 to 11008, HIP graph, one box), where its choice is 1.4% from the best of
 // all kernels in the geometric mean.  Skinny / best tile / split: down 4096 x
 // 11008, 57 rows 27.3 / 67.3 / 18.3, 256 rows 114 / 67 / 32.6; gate/up 2048 x
-// 4096, 128 rows 13.8 / 39.4 / 17.8; 11008 x 4096, 57 rows 38 / 40 / 31.
+// 4096, 128 rows 13.8 / 39.4 / 17.8; 11008 x 4096, 57 rows 38 / 40 / 27.
 // Without splits (`splits` false) the same choice among the rest.
 hxm_gemm_config default_w8_config(int epi, int64_t M, int64_t N, int64_t n_out, int64_t K,
                                   bool splits) {
-  static constexpr struct { double base, stage; } kCost[kNumW8Kernels] = {
-      {7.0, 0.94}, {7.0, 0.96}, {5.5, 0.53}, {6.0, 0.58}, {4.3, 0.37}};
-  constexpr double kStage2 = 0.70, kSplitBase = 9.2, kPlaneBytesPerUs = 6.2e6;
+  static constexpr struct { double base, stage, stage2, split_base; } kCost[kNumW8Kernels] = {
+      {7.0, 0.94, 0, 0}, {7.0, 0.96, 0, 0},      {5.5, 0.53, 0, 0},
+      {6.0, 0.58, 0, 0}, {4.3, 0.37, 0.70, 9.2}, {4.0, 0.33, 0.62, 8.5}};
+  constexpr double kPlaneBytesPerUs = 6.2e6;
   constexpr int64_t kCus = 256;
   const bool swiglu = epi == kEpiSwiglu;
   const auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
@@ -615,25 +618,26 @@ hxm_gemm_config default_w8_config(int epi, int64_t M, int64_t N, int64_t n_out, 
   const auto offer = [&](const hxm_gemm_config& c, double us) {
     if (us < best_us) best = c, best_us = us;
   };
-  const auto walk2 = [&](int64_t groups, int64_t stages) {
+  const auto walk2 = [&](int i, int64_t groups, int64_t stages) {
     const int64_t rem = groups % (2 * kCus);
     return static_cast<double>(stages) *
-           (groups / (2 * kCus) * kStage2 +
-            (rem == 0 ? 0.0 : rem <= kCus ? kCost[kW8PartEntry].stage : kStage2));
+           (groups / (2 * kCus) * kCost[i].stage2 +
+            (rem == 0 ? 0.0 : rem <= kCus ? kCost[i].stage : kCost[i].stage2));
   };
   for (int i = 0; i < kNumW8Kernels; ++i) {
     const hxm_gemm_config c = w8_kernel_config(i);
     const int64_t tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn), stages = ceil_div(K, c.bk);
+    const bool part = w8_split_valid(i, 2);
+    if (part && (c.bm == 64) != (M <= 64)) continue;
     if (!swiglu || w8_kernel_has_swiglu(i))
-      offer(c, kCost[i].base + (i == kW8PartEntry
-                                    ? walk2(tiles, stages)
+      offer(c, kCost[i].base + (part
+                                    ? walk2(i, tiles, stages)
                                     : static_cast<double>(ceil_div(tiles, kCus) * stages) *
                                           kCost[i].stage));
-    if (i != kW8PartEntry || !splits) continue;
-    for (int32_t s = 2; w8_split_valid(i, s) && tiles * s <= 2 * kCus && stages >= 4 * s; ++s) {
+    for (int32_t s = 2; splits && w8_split_valid(i, s) && tiles * s <= 2 * kCus && stages >= 4 * s; ++s) {
       hxm_gemm_config sc = c;
       sc.split_k = s;
-      offer(sc, kSplitBase + walk2(tiles * s, ceil_div(stages, s)) +
+      offer(sc, kCost[i].split_base + walk2(i, tiles * s, ceil_div(stages, s)) +
                     static_cast<double>(s * M) * w8_plane_ld(N) * 8 / kPlaneBytesPerUs);
     }
   }
@@ -864,7 +868,7 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
         static_cast<int>((K * 2 + bkb - 1) / bkb + plan.config.split_k - 1) / plan.config.split_k *
         static_cast<int>(bkb);
     q.plane_elems = M * ldp;
-    hipLaunchKernelGGL(kW8PartFns[sw ? 1 : 0],
+    hipLaunchKernelGGL(kW8PartFns[wi - kW8PartEntry][sw ? 1 : 0],
                        dim3(static_cast<unsigned>(plan.tiles), static_cast<unsigned>(S)),
                        dim3(e->threads), 0, stream, q);
     if ((st = check_launch("w8a16 split gemm")) != HXM_OK) return st;

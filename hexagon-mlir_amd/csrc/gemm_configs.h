@@ -29,5 +29,5 @@
 #define HXM_W8_CONFIG_LIST(X)                                                   \
   X(256, 256, 128, 3, 2, 2), X(256, 256, 128, 2, 2, 2),                          \
       X(256, 128, 128, 3, 2, 2), X(128, 256, 128, 4, 2, 2),                      \
-      X(128, 128, 128, 3, 2, 2)
+      X(128, 128, 128, 3, 2, 2), X(64, 128, 128, 4, 1, 2)
 #endif

@@ -1308,12 +1308,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
 
 typedef void (*gemm_fn)(GemmArgs);
 
-// The W8A16 K split (gemm_w8part.hip): kernels of entry kW8PartEntry of
-// HXM_W8_CONFIG_LIST that write fp32 partial planes ({kEpiW8Part, kEpiSwPart}),
+// The W8A16 K split (gemm_w8part.hip): kernels of the kW8PartEntries entries of
+// HXM_W8_CONFIG_LIST from kW8PartEntry on that write fp32 partial planes ({kEpiW8Part, kEpiSwPart}),
 // and the pass that adds the S planes ([S][M][ldp], plane order) and runs the
 // epilogue of g.
-constexpr int kW8PartEntry = 4;
-extern const gemm_fn kW8PartFns[2];
+constexpr int kW8PartEntry = 4, kW8PartEntries = 2;
+extern const gemm_fn kW8PartFns[kW8PartEntries][2];
 hxm_status launch_w8_reduce(int epi, const GemmArgs& g, const float* planes, int S, int64_t ldp,
                             hipStream_t stream);
 

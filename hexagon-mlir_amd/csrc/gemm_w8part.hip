@@ -1,4 +1,4 @@
-// K split of the W8A16 GEMMs: the 128x128 tile with workgroup row z taking one
+// K split of the W8A16 GEMMs: the 128x128 and 64x128 tiles with workgroup row z taking one
 // slice of K into an fp32 partial plane, and the pass that adds the planes.
 //
 // A call of few tiles is bound by the walk over K of each: at 57 rows the
@@ -8,14 +8,22 @@
 // workgroup: 18.3 us with the planes' write and read (S * M * N * 4 bytes each)
 // and the second launch.  512 x 1024 x 4096: 27.5 us unsplit, 14.5 in 6 slices;
 // 256 rows of hidden 11008, intermediate 2048, gate/up: 71.6, 32.6 in 4.
+//
+// Up to 64 rows the 64x128 tile takes the place of the 128x128 one: half the x
+// rows staged and half the MFMA work.  57 rows, 4096 -> 11008 gate/up in 2
+// slices 34.2, 27.0 us; the down projection in 8 slices 19.4, 18.0.
 #include "gemm_kernel.h"
 
 namespace hxm {
 
-static constexpr ConfigKey kKey = kW8Keys[kW8PartEntry];
-extern const gemm_fn kW8PartFns[2] = {
-    gemm_kernel<_Float16, kKey.bm, kKey.bn, kKey.bkb, kKey.st, kKey.wm, kKey.wn, kEpiW8Part>,
-    gemm_kernel<_Float16, kKey.bm, kKey.bn, kKey.bkb, kKey.st, kKey.wm, kKey.wn, kEpiSwPart>};
+template <int I, int EPI>
+static constexpr gemm_fn part_kernel() {
+  constexpr ConfigKey k = kW8Keys[kW8PartEntry + I];
+  return gemm_kernel<_Float16, k.bm, k.bn, k.bkb, k.st, k.wm, k.wn, EPI>;
+}
+extern const gemm_fn kW8PartFns[kW8PartEntries][2] = {
+    {part_kernel<0, kEpiW8Part>(), part_kernel<0, kEpiSwPart>()},
+    {part_kernel<1, kEpiW8Part>(), part_kernel<1, kEpiSwPart>()}};
 
 // One thread: four consecutive output columns of a row.  Plane rows are ldp
 // floats, a multiple of four; SwiGLU reads the gate channels and, 64 image rows

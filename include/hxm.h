@@ -98,7 +98,7 @@ typedef struct hxm_gemm_config {
                                S * M * N * 4 bytes, live in a library-owned
                                per-stream buffer kept until hxm_release_cache();
                                above 256 MiB the call is refused
-                               ("workspace-budget").  W8A16 GEMMs, 128x128 tile:
+                               ("workspace-budget").  W8A16 GEMMs, 64x128 and 128x128 tiles:
                                2 to 16, fp32 planes summed in order, also the
                                default of calls with few tiles and a long K
                                (where the planes cannot be had, as in a capture

@@ -39,10 +39,11 @@ def untouched(buf, M, N):
 
 @pytest.mark.parametrize("M,N,K,S", [(1, 1, 16, 2), (57, 333, 656, 2), (128, 128, 1024, 16),
                                      (129, 130, 2064, 5), (57, 258, 1040, 16), (300, 515, 720, 3)])
-@pytest.mark.parametrize("pad", [0, 3])
-def test_against_oracle(dev, M, N, K, S, pad):
-    print(f"w8 split M={M} N={N} K={K} S={S} pad={pad}", flush=True)
-    cfg = (128, 128, 64, 2, 2, 3, S)
+@pytest.mark.parametrize("tile,pad", [((128, 128, 64, 2, 2, 3), 0), ((128, 128, 64, 2, 2, 3), 3),
+                                      ((64, 128, 64, 1, 2, 4), 1)])
+def test_against_oracle(dev, M, N, K, S, tile, pad):
+    print(f"w8 split M={M} N={N} K={K} S={S} tile={tile} pad={pad}", flush=True)
+    cfg = tile + (S,)
     g, x, (W,), (s,) = operands(M, N, K)
     r = (4 * torch.randn(M, N, generator=g)).half()
     buf, y = padded(M, N, dev, pad)
