@@ -1,4 +1,6 @@
-// W8A16 weight-resident skinny GEMM / GEMV on gfx950 (M <= 16 per pass).
+// W8A16 weight-resident skinny GEMM / GEMV on gfx950 (M <= 16 per pass).  The
+// kernels here take the packed image and M = 1; plain weights at M > 1 go to the
+// skinny kernel (skinny_kernel.h).
 //
 // Reference semantics: an int8-weight linalg.matmul, which the reference's
 // engine refuses (qcom_hexagon_backend/include/hexagon/Dialect/Hmx/Transforms/
@@ -577,8 +579,8 @@ hxm_status hxm_gemv_w8a16(const void* x, int64_t ldx, const int8_t* W, int64_t l
   const int cb = !pk || M <= 4 || (N + 15) / 16 < kGemvCb3MinGroups ? 1 : 3;
   if ((st = check_grid("gemv_w8a16", (N + 16 * cb - 1) / (16 * cb), 512, (M + 15) / 16)) != HXM_OK)
     return st;
-  // M = 1 (and the plain [N, K] layout at every M, and the packed image at
-  // M <= 4 below kGemvPipeMinGroups): a 4096-wide K chunk (x rows fit LDS),
+  // M = 1 (and a plain [N, K] layout the skinny kernel left, and the packed
+  // image at M <= 4 below kGemvPipeMinGroups): a 4096-wide K chunk (x rows fit LDS),
   // so at K <= 4096 each wave issues all its weight loads at once and makes
   // one memory round trip.  Otherwise the packed image at M > 1 takes the
   // pipelined kernel, 512-wide chunks with the next chunk in flight.  The

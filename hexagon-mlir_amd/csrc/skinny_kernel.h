@@ -1,6 +1,6 @@
 #pragma once
-// Skinny MFMA matmuls on gfx950: at most 64 rows of A against the [N, K]
-// weight image.
+// Skinny MFMA matmuls on gfx950: up to 64 rows of A per workgroup (a call has
+// at most kSkinnyRowsMax) against the [N, K] image of B, or B as it is [K, N].
 //
 // What bounds such a call is the weight stream: each weight byte meets at
 // most 64 rows, far below the matrix cores' ratio.  The LDS-staged tiles
@@ -31,7 +31,8 @@
 // Gate/up + SwiGLU and down projection (hidden 4096, intermediate 11008),
 // against the 256-row tiles: 1 row 65.8 -> 14.1 and 94.7 -> 9.6 us, 16 rows
 // 66.2 -> 19.2 and 94.8 -> 13.3, 32 rows 66.6 -> 25.0 and 95.1 -> 19.3, 57
-// rows 67.5 -> 40.7 and 96.5 -> 30.4 (one box).
+// rows 67.5 -> 40.7 and 96.5 -> 30.4 (one box; from 33 rows on a K split of the
+// 64x128 tile can be the shorter one, 27.0 and 18.0 there: default_w8_config).
 #include <type_traits>
 
 #include "gemm_kernel.h"
