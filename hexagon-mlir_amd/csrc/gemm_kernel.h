@@ -1100,7 +1100,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
   }
 
   // General path: accumulate, unaligned rows, edge tiles whose runs may
-  // straddle N.
+  // straddle N.  A run inside C is one vector access whatever its alignment
+  // (element by element only where it straddles N): the stores of a run were
+  // this path's whole cost.  bf16 2772 x 4091 x 192 (128x128, two stages) 24.6
+  // -> 18.4 us, int8 27.3 -> 18.0, bf16 4096 x 3073 x 256 25.9 -> 18.6; aligned
+  // rows of 4096 take 11.0 and 11.9.
+  typedef v8f16 any8f16 __attribute__((aligned(2)));
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
     stage_block(i);
@@ -1137,6 +1142,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
         _Float16* c = static_cast<_Float16*>(g.C) + static_cast<int64_t>(m) * g.ldc + n;
         if (g.vec8_store && n + 8 <= g.N) {
           __builtin_nontemporal_store(h, reinterpret_cast<v8f16*>(c));  // C is not re-read here
+        } else if (n + 8 <= g.N) {
+          *reinterpret_cast<any8f16*>(c) = h;
         } else {
           for (int e = 0; e < 8 && n + e < g.N; ++e) c[e] = h[e];
         }
@@ -1161,8 +1168,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
         v8f16 rv = {};
         if constexpr (EPI == kEpiW8Res) {
           const _Float16* r = g.residual + static_cast<int64_t>(m) * g.ldr + n;
-          if (g.res_vec8 && n + 8 <= g.N)
-            rv = *reinterpret_cast<const v8f16*>(r);
+          if (n + 8 <= g.N)
+            rv = *reinterpret_cast<const any8f16*>(r);
           else
             for (int e = 0; e < 8 && n + e < g.N; ++e) rv[e] = r[e];
         }
@@ -1180,6 +1187,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
         _Float16* c = static_cast<_Float16*>(g.C) + static_cast<int64_t>(m) * g.ldc + n;
         if (g.vec8_store && n + 8 <= g.N) {
           store_out8<EPI>(h, c);
+        } else if (n + 8 <= g.N) {
+          *reinterpret_cast<any8f16*>(c) = h;
         } else {
           for (int e = 0; e < 8 && n + e < g.N; ++e) c[e] = h[e];
         }
@@ -1220,6 +1229,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
         _Float16* c = static_cast<_Float16*>(g.C) + static_cast<int64_t>(m) * g.ldc + o;
         if (g.vec8_store && o + 8 <= g.n_out) {
           store_out8<EPI>(h, c);
+        } else if (o + 8 <= g.n_out) {
+          *reinterpret_cast<any8f16*>(c) = h;
         } else {
           for (int e = 0; e < 8 && o + e < g.n_out; ++e) c[e] = h[e];
         }
@@ -1246,16 +1257,20 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
       const int m = mw + i * 32 + row, n = nw + col;
       if (m >= g.M || n >= g.N) continue;
       const int64_t off = static_cast<int64_t>(m) * g.ldc + n;
-      const bool full = g.vec_store && n + 4 <= g.N;
+      const bool full = n + 4 <= g.N;
+      typedef v4u32_t any4u32 __attribute__((aligned(4)));
+      typedef v4f32 any4f32 __attribute__((aligned(4)));
+      typedef v4f16_t any4f16 __attribute__((aligned(2)));
+      typedef v4bf16_t any4bf16 __attribute__((aligned(2)));
       if constexpr (EPI == kEpiI32) {
         int32_t* c = static_cast<int32_t*>(g.C) + off;
         v4u32_t r = __builtin_bit_cast(v4u32_t, w);
         if (full) {
           if (g.accumulate) {
-            r += *reinterpret_cast<const v4u32_t*>(c);
-            *reinterpret_cast<v4u32_t*>(c) = r;
+            r += *reinterpret_cast<const any4u32*>(c);
+            *reinterpret_cast<any4u32*>(c) = r;
           } else {
-            __builtin_nontemporal_store(r, reinterpret_cast<v4u32_t*>(c));
+            *reinterpret_cast<any4u32*>(c) = r;  // lines shared with other runs: L2 merges them
           }
         } else {
           for (int e = 0; e < 4 && n + e < g.N; ++e)
@@ -1266,8 +1281,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
         if (g.out_dtype == HXM_F32) {
           float* c = static_cast<float*>(g.C) + off;
           if (full) {
-            if (g.accumulate) r += *reinterpret_cast<const v4f32*>(c);
-            *reinterpret_cast<v4f32*>(c) = r;
+            if (g.accumulate) r += *reinterpret_cast<const any4f32*>(c);
+            *reinterpret_cast<any4f32*>(c) = r;
           } else {
             for (int e = 0; e < 4 && n + e < g.N; ++e) c[e] = g.accumulate ? c[e] + r[e] : r[e];
           }
@@ -1275,12 +1290,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
           _Float16* c = static_cast<_Float16*>(g.C) + off;
           if (full) {
             if (g.accumulate) {
-              const v4f16_t o = *reinterpret_cast<const v4f16_t*>(c);
+              const v4f16_t o = *reinterpret_cast<const any4f16*>(c);
               for (int e = 0; e < 4; ++e) r[e] += static_cast<float>(o[e]);
             }
             v4f16_t h;
             for (int e = 0; e < 4; ++e) h[e] = static_cast<_Float16>(r[e]);
-            *reinterpret_cast<v4f16_t*>(c) = h;
+            *reinterpret_cast<any4f16*>(c) = h;
           } else {
             for (int e = 0; e < 4 && n + e < g.N; ++e)
               c[e] = static_cast<_Float16>(g.accumulate ? r[e] + static_cast<float>(c[e]) : r[e]);
@@ -1289,12 +1304,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g0) {
           __bf16* c = static_cast<__bf16*>(g.C) + off;
           if (full) {
             if (g.accumulate) {
-              const v4bf16_t o = *reinterpret_cast<const v4bf16_t*>(c);
+              const v4bf16_t o = *reinterpret_cast<const any4bf16*>(c);
               for (int e = 0; e < 4; ++e) r[e] += static_cast<float>(o[e]);
             }
             v4bf16_t h;
             for (int e = 0; e < 4; ++e) h[e] = static_cast<__bf16>(r[e]);
-            *reinterpret_cast<v4bf16_t*>(c) = h;
+            *reinterpret_cast<any4bf16*>(c) = h;
           } else {
             for (int e = 0; e < 4 && n + e < g.N; ++e)
               c[e] = static_cast<__bf16>(g.accumulate ? r[e] + static_cast<float>(c[e]) : r[e]);
