@@ -88,25 +88,36 @@ const KernelEntry* find_kernel(const hxm_gemm_config& c, int32_t dt) {
 //   f16 128 x 4096 x 4096: 64x64 19 / 16.9, 128x64 20 / 20.1 (before: 31.8)
 // The deeper prefetch of the small tiles is what they gain: with two stages a
 // 64x64 tile has 32 KiB a CU in flight and waits for every round trip.
+//
+// An N off the vector boundary takes the general epilogue (`ragged` more a
+// workgroup), where the large tiles' one wave per SIMD waits for each run's
+// store: bf16 2772 x 4091 x 192 256x256 35.8, 256x128 27.9, 128x128 21.9, 64x64
+// 21.1, 128x128 of two stages (two workgroups a CU) 18.4.  The last is offered
+// for such an N only, where two fit and K is at most 16 stages (1024: 36.0 us
+// against 38.1; 2048: 59.2 against 57.8).
 hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt) {
   struct Tile {
     int bm, bn, stages, occ;
-    double fixed, stage_lo, stage_hi;
+    double fixed, stage_lo, stage_hi, ragged;
   };
-  static const Tile tiles[] = {{256, 256, 2, 1, 5.0, 1.10, 1.55},
-                               {256, 128, 3, 1, 4.0, 0.75, 0.93},
-                               {128, 128, 3, 1, 3.5, 0.45, 0.57},
-                               {128, 64, 4, 1, 3.3, 0.22, 0.36},
-                               {64, 64, 4, 2, 2.6, 0.19, 0.44}};
+  static const Tile tiles[] = {{256, 256, 2, 1, 5.0, 1.10, 1.55, 23.0},
+                               {256, 128, 3, 1, 4.0, 0.75, 0.93, 8.0},
+                               {128, 128, 3, 1, 3.5, 0.45, 0.57, 2.8},
+                               {128, 128, 2, 2, 4.0, 0.14, 0.94, 4.2},
+                               {128, 64, 4, 1, 3.3, 0.22, 0.36, 1.5},
+                               {64, 64, 4, 2, 2.6, 0.19, 0.44, 1.0}};
+  const bool ragged = N % 4 != 0;
   const double kt = static_cast<double>(ceil_div(K * elem_bytes(dt), 128));
   constexpr double kCus = 256;
   const Tile* best = nullptr;
   double best_us = 0;
   for (const Tile& t : tiles) {
     const double n = static_cast<double>(ceil_div(M, t.bm)) * static_cast<double>(ceil_div(N, t.bn));
+    if (t.bm == 128 && t.stages == 2 && !(ragged && n > kCus && kt <= 16)) continue;
     const double rounds = std::max(1.0, std::ceil(n / (kCus * t.occ)));
     const double load = n / (rounds * kCus * t.occ);
-    const double us = rounds * (t.fixed + kt * (t.stage_lo + (t.stage_hi - t.stage_lo) * load));
+    const double us = rounds * (t.fixed + (ragged ? t.ragged : 0.0) +
+                                kt * (t.stage_lo + (t.stage_hi - t.stage_lo) * load));
     if (!best || us < best_us) best = &t, best_us = us;
   }
   hxm_gemm_config c{best->bm, best->bn, 128 / elem_bytes(dt), 2, 2, best->stages, 1};

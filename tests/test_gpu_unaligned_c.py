@@ -79,3 +79,23 @@ def test_w8a16_rows_off_the_vector_boundary(M, N, residual):
     ops.gemm_w8a16(x, W[:N], s[:N], out=view, config=cfg,
                    residual=r[:, :N].contiguous() if residual else None)
     _check(buf, view, want, 1)
+
+
+# The default tile where N is off the vector boundary: two-stage 128x128 from
+# 257 tiles to 16 stages of K, not at 256 tiles nor beyond 16 stages.
+@pytest.mark.parametrize("M,N,kb,two_stage", [(2050, 2011, 336, True), (1990, 2010, 400, False),
+                                              (2050, 2011, 2048, True), (2050, 2011, 2064, False)])
+@pytest.mark.parametrize("i8", [False, True])
+def test_default_tile_at_ragged_n(M, N, kb, two_stage, i8):
+    g = torch.Generator(device="cuda").manual_seed(7)
+    if i8:
+        A, B = (torch.randint(-127, 128, (r, kb), generator=g, device="cuda", dtype=torch.int8)
+                for r in (M, N))
+    else:
+        A, B = (torch.randn(r, kb // 2, generator=g, device="cuda").half() for r in (M, N))
+    f = ops.gemm_i8 if i8 else ops.matmul
+    C = f(A, B, b_layout="nk")
+    c = ops.last_plan()["config"]
+    assert ((c[0], c[1], c[5]) == (128, 128, 2)) == two_stage
+    assert torch.equal(C, f(A, B, b_layout="nk", config=(256, 256, 128 if i8 else 64,
+                                                         2, 2, 2, 1)))
