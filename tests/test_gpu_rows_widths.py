@@ -70,3 +70,36 @@ def test_many_short_rows(dev, name, nv):
     cols = nv * (4 if name == "f32" else 8)
     for c in (max(1, cols - 1), cols, cols + 1):
         check(dev, name, 2051, c)
+
+
+def extreme_rows(name, cols, g):
+    """Softmax rows whose maximum is large: wholly masked ones (the lowest value,
+    -1e10), one peak near the largest value, and steps of one unit or less at
+    growing offsets, where a scaled maximum rounds by more than the steps."""
+    big = torch.finfo(TDT[name]).max
+    ten = 1e10 if name != "f16" else 6e4
+    x = [torch.full((cols,), v) for v in (-big, -ten, ten, big)]
+    x.append(2 * torch.randn(cols, generator=g))
+    x[-1][cols // 3] = big * 0.88
+    x.append(torch.where(torch.arange(cols) % 3 == 0, big, -big))
+    steps = -torch.randint(0, 40, (cols,), generator=g) * 0.5
+    x += [steps + off for off in (1e3, -1e3, 4e4, -4e4)]
+    if name != "f16":
+        x += [steps + off for off in (4194300.0, -4194300.0, 4194400.0, -4194400.0)]
+        x += [v * (1 + steps / 3e7) for v in (3.5e9, -3.5e9, 2e38, -2e38)]
+    return torch.stack(x).to(TDT[name])
+
+
+@pytest.mark.parametrize("nv", [1, 16, 48, 63] + list(EDGES))
+@pytest.mark.parametrize("name", ["f16", "bf16", "f32"])
+def test_softmax_of_large_maxima(dev, name, nv):
+    for c in (-1, 0, 1):
+        cols = nv * (4 if name == "f32" else 8) + c
+        x = extreme_rows(name, cols, torch.Generator().manual_seed(cols))
+        if nv < 64:
+            x = x.repeat(2048 // len(x) + 1, 1)          # four short rows to a wave
+        print(f"{name} {tuple(x.shape)}", flush=True)
+        y = ops.softmax(x.to(dev)).float().cpu().numpy()
+        ref = orc.to_f32(orc.softmax_rows(bits(x, name), name), name)
+        np.testing.assert_allclose(y, ref, **TOL[name])
+        np.testing.assert_allclose(y.sum(1, dtype=np.float64), 1, rtol=1e-2)
