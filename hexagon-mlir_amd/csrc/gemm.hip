@@ -708,7 +708,8 @@ hxm_status plan_gemm_w8(int32_t op, int epi, int64_t M, int64_t N, int64_t n_out
   if (cfg && cfg->bm) {
     c = *cfg;
     p->source = HXM_SOURCE_CALLER;
-  } else if (lookup_tuned(op, M, sw ? n_out : N, K, &c)) {
+  } else if (lookup_tuned(op, M, sw ? n_out : N, K, &c) &&
+             (splits || c.split_k <= 1 || c.split_k == HXM_STREAM_K)) {
     p->source = HXM_SOURCE_TUNED;
   } else {
     c = default_w8_config(epi, M, N, n_out, K, splits);
@@ -805,11 +806,14 @@ hxm_status run_gemm_w8(int epi, int32_t op, const void* x, int64_t ldx, const in
   if (M == 0 || N == 0) return ok();
   void* planes = nullptr;
   if (e && w8_split_valid(static_cast<int>(e - kW8Kernels), plan.config.split_k)) {
-    // An untuned call works on any stream at any time: where the planes cannot
-    // be had (a capture that would have to grow them, no memory) it runs the
-    // best kernel without them.
-    st = stream_workspace(stream, static_cast<size_t>(plan.workspace_bytes), &planes, kWsSplitK);
-    if (st != HXM_OK && plan.source == HXM_SOURCE_DEFAULT)
+    // A split that the library chose is not captured: the graph would hold the
+    // capture stream's planes, which a replay beside another graph's, or beside
+    // an eager call of that stream, would overwrite.  There, and where the
+    // planes cannot be had, the call runs the best kernel without them.
+    const bool chosen = plan.source != HXM_SOURCE_CALLER;
+    if (!chosen || !stream_capturing(stream))
+      st = stream_workspace(stream, static_cast<size_t>(plan.workspace_bytes), &planes, kWsSplitK);
+    if (chosen && !planes)
       st = plan_gemm_w8(op, epi, M, N, n_out, K, cfg, false, &plan, &e);
     if (st != HXM_OK) return st;
   }

@@ -24,7 +24,12 @@
  *     per-stream workspace (f32 operands, a [K,N] B, a K split) needs it
  *     already large enough: one call of the shape on the stream before the
  *     capture grows it (it is kept until hxm_release_cache, also past a later
- *     growth once a graph has captured it).
+ *     growth once a graph has captured it).  Such a graph holds the workspace
+ *     of the stream it was captured on: it must not run at the same time as
+ *     another graph captured on that stream, nor as other calls on that
+ *     stream, wherever it is replayed.  A call without a config captures no
+ *     W8A16 K split (the best unsplit kernel instead), so untuned W8A16 GEMMs
+ *     need no workspace and their graphs stand alone.
  *   - numerics: fp16/bf16 products accumulate in fp32 and are rounded once
  *     to the output dtype; int8 products accumulate exactly in int32.
  *   - host threads: entries may run at the same time on several host
@@ -101,9 +106,9 @@ typedef struct hxm_gemm_config {
                                ("workspace-budget").  W8A16 GEMMs, 64x128 and 128x128 tiles:
                                2 to 16, fp32 planes summed in order, also the
                                default of calls with few tiles and a long K
-                               (where the planes cannot be had, as in a capture
-                               that would have to grow them, an untuned call runs
-                               unsplit).
+                               (in a capture, and where there is no memory for the
+                               planes, a call without a config runs unsplit; the
+                               two sum in different orders).
                                HXM_STREAM_K: the W8A16 GEMMs' stream-K mode
                                (below) */
 } hxm_gemm_config;

@@ -6,7 +6,9 @@ import numpy as np
 import pytest
 import torch
 
+import hxm
 import hxm.ops as ops
+from hxm import search as S
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -69,37 +71,89 @@ def test_against_oracle(dev, M, N, K, S, tile, pad):
     assert untouched(buf, M, N)
 
 
-def test_untuned_choice_and_capture(dev):
-    """57 rows of a long K are split when untuned.  A capture on a stream that
-    has the planes replays the eager call's bits, also after the planes have
-    grown; on a stream without them it runs unsplit instead of being refused."""
+def test_untuned_choice_and_capture(dev, tmp_path):
+    """57 rows of a long K are split when untuned, and by a tuned winner that is
+    a split.  A capture of either runs unsplit, also on a stream that has the
+    planes: its graph holds no workspace, so graphs captured on one stream
+    replay at once, beside an eager split call of that stream."""
     g, x, (W,), (s,) = operands(57, 1024, 8192)
+    xs = [x.to(dev), torch.randn(57, 8192, generator=g).half().to(dev)]
+    W, s = W.to(dev), s.to(dev)
+    ys = [torch.empty(57, 1024, dtype=torch.float16, device=dev) for _ in xs]
+    eager = torch.empty_like(ys[0])
+    hxm.lib.hxm_tune_cache_clear()
+    cache = tmp_path / "tune.txt"
+    S.tune_cache_save(str(cache))                    # this build's header
+    with open(cache, "a") as f:
+        f.write("16 57 1024 8192 128 128 64 2 2 3 4 3\n")
+    others = [torch.cuda.Stream(), torch.cuda.Stream()]
+    try:
+        for tuned in (False, True):
+            print(f"capture tuned={tuned}", flush=True)
+            if tuned:
+                assert S.tune_cache_load(str(cache)) == 1
+            warm = torch.cuda.Stream()
+            with torch.cuda.stream(warm):
+                ops.gemm_w8a16(xs[1], W, s, out=eager)
+            plan = ops.last_plan()
+            assert plan["source"] == ("tuned" if tuned else "default")
+            assert plan["config"][6] > 1 and plan["workspace_bytes"] > 0
+            torch.cuda.synchronize()
+            split = eager.clone()
+            graphs = []
+            for xi, yi in zip(xs, ys):
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=warm):
+                    ops.gemm_w8a16(xi, W, s, out=yi)
+                plan = ops.last_plan()
+                assert plan["config"][6] <= 1 and plan["workspace_bytes"] == 0
+                graph.replay()
+                torch.cuda.synchronize()
+                graphs.append(graph)
+            want = [y.clone() for y in ys]
+            for xi, w in zip(xs, want):
+                ref = orc.f16_bits_to_f32(orc.gemm_w8a16(bits(xi), W.cpu().numpy(),
+                                                         s.cpu().numpy()))
+                np.testing.assert_allclose(w.float().cpu().numpy(), ref, **TOL)
+            for rep in range(20):
+                for y in ys + [eager]:
+                    y.fill_(-7.0)
+                torch.cuda.synchronize()
+                for graph, st in zip(graphs, others):
+                    with torch.cuda.stream(st):
+                        graph.replay()
+                with torch.cuda.stream(warm):
+                    ops.gemm_w8a16(xs[1], W, s, out=eager)
+                torch.cuda.synchronize()
+                for y, w in zip(ys, want):
+                    assert torch.equal(y, w), rep
+                assert torch.equal(eager, split), rep
+    finally:
+        hxm.lib.hxm_tune_cache_clear()
+
+
+def test_requested_split_in_a_graph(dev):
+    """A split asked for by config is captured with the stream's planes: its
+    replays give the eager call's bits, also after the planes have grown."""
+    cfg = (128, 128, 64, 2, 2, 3, 4)
+    _, x, (W,), (s,) = operands(57, 1024, 8192)
     x, W, s = x.to(dev), W.to(dev), s.to(dev)
     y = torch.empty(57, 1024, dtype=torch.float16, device=dev)
-    warm, fresh = torch.cuda.Stream(), torch.cuda.Stream()
+    warm = torch.cuda.Stream()
     with torch.cuda.stream(warm):
-        ops.gemm_w8a16(x, W, s, out=y)
-    plan = ops.last_plan()
-    assert plan["config"][6] > 1 and plan["workspace_bytes"] > 0
+        ops.gemm_w8a16(x, W, s, out=y, config=cfg)
     torch.cuda.synchronize()
     want = y.clone()
-    graphs = []
-    for st, split in ((warm, True), (fresh, False)):
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=st):
-            ops.gemm_w8a16(x, W, s, out=y)
-        assert (ops.last_plan()["config"][6] > 1) == split
-        graphs.append(graph)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=warm):
+        ops.gemm_w8a16(x, W, s, out=y, config=cfg)
+    assert ops.last_plan()["config"] == cfg
     big = torch.randn(512, 8192, device=dev).half()
     with torch.cuda.stream(warm):                    # grows that stream's planes
-        ops.gemm_w8a16(big, W, s, config=(128, 128, 64, 2, 2, 3, 16))
+        ops.gemm_w8a16(big, W, s, config=cfg[:6] + (16,))
     for rep in range(3):
-        for graph, exact in zip(graphs, (True, False)):
-            y.fill_(-7.0)
-            torch.cuda.synchronize()
-            graph.replay()
-            torch.cuda.synchronize()
-            if exact:
-                assert torch.equal(y, want), rep
-            else:
-                torch.testing.assert_close(y, want, rtol=1e-2, atol=1e-3)
+        y.fill_(-7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), rep
