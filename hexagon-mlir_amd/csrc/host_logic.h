@@ -63,6 +63,16 @@ inline bool split_planes_fit(int64_t slices, int64_t M, int64_t N, int64_t max_b
   return M <= max_bytes / 4 / slices / N;
 }
 
+// Whether the tuner holds a candidate's output to the float tolerance instead
+// of the control's bits.  Another kernel family (other_kernel: the direct
+// small-output or the skinny kernel on one side) or K split adds fp32 sums in
+// another order; integer sums are exact in any order, and their words, read as
+// pairs of halves, would all agree up to about 5100.
+inline bool verify_by_tolerance(int32_t op, bool other_kernel, int32_t split,
+                                int32_t control_split) {
+  return op != HXM_I8 && (other_kernel || split != control_split);
+}
+
 // Stream-K layout of an int8-weight GEMM launch of `ntiles` tiles of KT K
 // stages each on `cus` CUs (one workgroup per CU): the first dp tiles, whole
 // rounds, run one per workgroup; the rest (tiles = ntiles mod cus) are cut

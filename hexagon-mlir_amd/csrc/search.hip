@@ -412,10 +412,12 @@ hxm_status tune_core(const TuneSpec& sp, int32_t reps, hxm_gemm_config* best, ch
       // The direct-load small-output kernel, the skinny kernel (partial sums
       // of its waves) and the float K splits and stream-K tiles (fp32 partial
       // sums added across workgroups) sum in another order than the staged
-      // one-workgroup tiles: checked within the float tolerance.
-      if (is_small_gemm_config(cands[i]) != is_small_gemm_config(control) ||
-          is_skinny_config(cands[i]) != is_skinny_config(control) ||
-          (op != HXM_I8 && cands[i].split_k != control.split_k))
+      // one-workgroup tiles: checked within the float tolerance.  int8 outputs
+      // are compared word for word whatever the kernels.
+      if (verify_by_tolerance(op,
+                              is_small_gemm_config(cands[i]) != is_small_gemm_config(control) ||
+                                  is_skinny_config(cands[i]) != is_skinny_config(control),
+                              cands[i].split_k, control.split_k))
         count_far_kernel<<<1024, 256, 0, s>>>(static_cast<const uint32_t*>(C),
                                               (ldc * out_eb) / 4, ref, M, row_words,
                                               op == HXM_BF16, bad);

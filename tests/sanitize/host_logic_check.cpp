@@ -229,6 +229,16 @@ int main() {
     for (int v : segs) most = std::max<int64_t>(most, v);
     CHECK(most == L.maxseg, "maxseg %d, most segments %lld", L.maxseg, (long long)most);
   }
+  // The tuner's check: int8 outputs are always compared bit for bit.
+  for (int32_t op : {int(HXM_I8), int(HXM_F16), int(HXM_BF16), int(HXM_OP_W8A16),
+                     int(HXM_OP_W8A16_SWIGLU)})
+    for (bool other : {false, true})
+      for (int32_t s : {1, 2, 16, HXM_STREAM_K})
+        for (int32_t c : {1, 2, 16, HXM_STREAM_K})
+          CHECK(hxm::verify_by_tolerance(op, other, s, c) ==
+                    (op != HXM_I8 && (other || s != c)),
+                "verify_by_tolerance op %d other %d splits %d %d", op, other, s, c);
+
   hxm::StreamKLayout L0;
   CHECK(!hxm::stream_k_layout(0, 4, 256, &L0) && !hxm::stream_k_layout(10, 0, 256, &L0) &&
             !hxm::stream_k_layout(10, 4, 0, &L0) && !hxm::stream_k_layout(512, 4, 256, &L0) &&

@@ -175,3 +175,23 @@ def test_tune_calibrated_repetitions_and_the_cost_model(dev):
     assert rep["champion"] is not None and not cfgs[rep["champion"]]["pruned"]
     C = ops.gemm_i8(A, B, b_layout="nk").cpu().numpy()
     assert np.array_equal(C, orc.gemm_i8(A.cpu().numpy(), B.cpu().numpy(), b_nk=True))
+
+
+def test_int8_candidates_equal_the_skinny_control_bit_for_bit(dev):
+    """Few rows: the control is the skinny kernel; the tiles and their K splits
+    must reproduce its int32 words exactly (sums here stay small, where words
+    read as floats would all be near each other)."""
+    import hxm
+    M, N, K = 17, 512, 2048
+    g = torch.Generator().manual_seed(7)
+    A = torch.randint(0, 2, (M, K), generator=g, dtype=torch.int8).to(dev)
+    B = torch.randint(0, 2, (N, K), generator=g, dtype=torch.int8).to(dev)
+    out = torch.empty(M, N, dtype=torch.int32, device=dev)
+    try:
+        _, rep = ops.tune_gemm(A, B, out, reps=3)
+        assert rep["configs"][rep["control"]]["tiles"][:2] == [16, 16]
+        measured = [c for c in rep["configs"] if c["q50"] is not None]
+        assert len(measured) > 5 and all(c["verified"] for c in measured)
+        assert any(c["split_k"] > 1 for c in measured)
+    finally:
+        hxm.lib.hxm_tune_cache_clear()
