@@ -95,17 +95,30 @@ const KernelEntry* find_kernel(const hxm_gemm_config& c, int32_t dt) {
 // 21.1, 128x128 of two stages (two workgroups a CU) 18.4.  The last is offered
 // for such an N only, where two fit and K is at most 16 stages (1024: 36.0 us
 // against 38.1; 2048: 59.2 against 57.8).
-hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt) {
+//
+// An accumulating call takes the general epilogue at every N and reads each run
+// of C before it can store it (`rmw` more a workgroup).  What hides that wait is
+// other workgroups of the CU, so both two-stage tiles are offered: 64x64 up to 16
+// stages, and 128x128 up to 32 where its last round puts two on a CU (a tile left
+// alone there walks K at the three-stage one's pace or slower: int8 3100 x 3500 x
+// 4000, 700 tiles, 85.2 us against 70.5 for 256x256).  The choice without the
+// read / with it (us, one box): f16 1500 x 2047 x 512 22.3 / 64x64 12.9; 2772 x
+// 4096 x 192 35.5 / 64x64 20.5; 4096 x 4096 x 1024 66.8 / 128x128 55.2; int8 2000
+// x 4000 x 2048 31.3 / 128x128 28.0.  Fitted to 138 calls (four operand and
+// output types, seven tiles each), where it is 0.4% from the best of them in the
+// geometric mean.
+hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt, bool accumulate) {
   struct Tile {
     int bm, bn, stages, occ;
-    double fixed, stage_lo, stage_hi, ragged;
+    double fixed, stage_lo, stage_hi, ragged, rmw;
   };
-  static const Tile tiles[] = {{256, 256, 2, 1, 5.0, 1.10, 1.55, 23.0},
-                               {256, 128, 3, 1, 4.0, 0.75, 0.93, 8.0},
-                               {128, 128, 3, 1, 3.5, 0.45, 0.57, 2.8},
-                               {128, 128, 2, 2, 4.0, 0.14, 0.94, 4.2},
-                               {128, 64, 4, 1, 3.3, 0.22, 0.36, 1.5},
-                               {64, 64, 4, 2, 2.6, 0.19, 0.44, 1.0}};
+  static const Tile tiles[] = {{256, 256, 2, 1, 5.0, 1.10, 1.55, 23.0, 20.0},
+                               {256, 128, 3, 1, 4.0, 0.75, 0.93, 8.0, 9.0},
+                               {128, 128, 3, 1, 3.5, 0.45, 0.57, 2.8, 3.0},
+                               {128, 128, 2, 2, 4.0, 0.14, 0.94, 4.2, 4.0},
+                               {128, 64, 4, 1, 3.3, 0.22, 0.36, 1.5, 1.3},
+                               {64, 64, 4, 2, 2.6, 0.19, 0.44, 1.0, 1.1},
+                               {64, 64, 2, 5, 2.2, 0.29, 0.87, 0.5, 0.6}};
   const bool ragged = N % 4 != 0;
   const double kt = static_cast<double>(ceil_div(K * elem_bytes(dt), 128));
   constexpr double kCus = 256;
@@ -113,10 +126,14 @@ hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt) {
   double best_us = 0;
   for (const Tile& t : tiles) {
     const double n = static_cast<double>(ceil_div(M, t.bm)) * static_cast<double>(ceil_div(N, t.bn));
-    if (t.bm == 128 && t.stages == 2 && !(ragged && n > kCus && kt <= 16)) continue;
+    if (t.bm == 128 && t.stages == 2 &&
+        !(accumulate ? kt <= 32 && std::fmod(n - 1, 2 * kCus) >= kCus
+                     : ragged && n > kCus && kt <= 16))
+      continue;
+    if (t.bm == 64 && t.stages == 2 && !(accumulate && kt <= 16)) continue;
     const double rounds = std::max(1.0, std::ceil(n / (kCus * t.occ)));
     const double load = n / (rounds * kCus * t.occ);
-    const double us = rounds * (t.fixed + (ragged ? t.ragged : 0.0) +
+    const double us = rounds * (t.fixed + (ragged ? t.ragged : 0.0) + (accumulate ? t.rmw : 0.0) +
                                 kt * (t.stage_lo + (t.stage_hi - t.stage_lo) * load));
     if (!best || us < best_us) best = &t, best_us = us;
   }
@@ -299,8 +316,8 @@ thread_local bool g_has_last_plan = false;
 // plan's op, `epi` the epilogue, `extra_ws` workspace the caller adds (the
 // f32 operand images).  The plan is also kept as this thread's last plan.
 hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64_t M,
-                     int64_t N, int64_t K, const hxm_gemm_config* cfg, int64_t extra_ws,
-                     hxm_plan* p, const KernelEntry** entry) {
+                     int64_t N, int64_t K, bool accumulate, const hxm_gemm_config* cfg,
+                     int64_t extra_ws, hxm_plan* p, const KernelEntry** entry) {
   *p = hxm_plan{};
   p->op = op;
   p->m = M, p->n = N, p->k = K;
@@ -319,7 +336,7 @@ hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64
   } else {
     c = epi == kEpiFloat && small_gemm_fits(M, N, K, table) ? small_gemm_config()
         : skinny_default(table, epi, M, N, K)                 ? skinny_config()
-                                                             : default_config(M, N, K, table);
+                                              : default_config(M, N, K, table, accumulate);
     p->source = HXM_SOURCE_DEFAULT;
   }
   p->config = c;
@@ -425,7 +442,8 @@ static hxm_status run_gemm_with(int32_t op, int32_t ab_dtype, int epi, const voi
   const int64_t eb = dtype_bytes(ab_dtype);
   const KernelEntry* e = nullptr;
   hxm_plan plan;
-  hxm_status st = plan_gemm(op, ab_dtype, epi, b_layout, M, N, K, cfg, extra_ws, &plan, &e);
+  hxm_status st = plan_gemm(op, ab_dtype, epi, b_layout, M, N, K, accumulate != 0, cfg, extra_ws,
+                            &plan, &e);
   if (st != HXM_OK) return st;
   // Caller-provided planes (the allocation-free entry's static array): the
   // call takes no library workspace, and its plan record says so.
@@ -971,7 +989,7 @@ hxm_status hxm_plan_matmul(int64_t M, int64_t N, int64_t K, int32_t a_dtype,
   const hxm_plan saved = g_last_plan;
   const bool had = g_has_last_plan;
   const hxm_status st = plan_gemm(a_dtype, table, epi, a_dtype == HXM_F32 ? HXM_B_NK : b_layout,
-                                  M, N, kk, cfg, extra, p, nullptr);
+                                  M, N, kk, false, cfg, extra, p, nullptr);
   g_last_plan = saved;
   g_has_last_plan = had;
   p->k = K;
@@ -1018,8 +1036,8 @@ static hxm_status matmul_f32(const float* A, int64_t lda, const float* B, int64_
   hxm_status st = HXM_OK;
   const int64_t a_bytes = (M * kp * 2 + 255) / 256 * 256, img_bytes = a_bytes + N * kp * 2;
   hxm_plan plan;
-  if ((st = plan_gemm(HXM_F32, HXM_F16, kEpiFloat, HXM_B_NK, M, N, kp, cfg, img_bytes, &plan,
-                      nullptr)) != HXM_OK)
+  if ((st = plan_gemm(HXM_F32, HXM_F16, kEpiFloat, HXM_B_NK, M, N, kp, accumulate != 0, cfg,
+                      img_bytes, &plan, nullptr)) != HXM_OK)
     return st;
   if ((st = require_device(nullptr)) != HXM_OK) return st;
   if (M == 0 || N == 0 || (K == 0 && accumulate)) return ok();

@@ -35,7 +35,7 @@ hxm_status run_gemm(int32_t op, int32_t ab_dtype, int epi, const void* A,
                     int32_t out_dtype, int32_t accumulate, const float* rs,
                     const float* cs, const hxm_gemm_config* cfg,
                     hipStream_t stream);
-hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt);
+hxm_gemm_config default_config(int64_t M, int64_t N, int64_t K, int32_t dt, bool accumulate);
 int num_w8_kernels();
 hxm_gemm_config w8_kernel_config(int i);
 bool w8_kernel_has_swiglu(int i);
@@ -895,7 +895,7 @@ hxm_status hxm_tune_gemm(int32_t op, const void* A, int64_t lda, const void* B,
   sort_configs(&sp.cands);
   sp.control = small ? small_gemm_config()
                : skinny_default(op, epi, M, N, K) ? skinny_config()
-                                             : default_config(M, N, K, op);
+                                             : default_config(M, N, K, op, false);
   if (skinny_fits(M, N, K)) sp.cands.insert(sp.cands.begin(), skinny_config());
   sp.canary = hxm_gemm_config{32, 32, static_cast<int32_t>(op == HXM_I8 ? 128 : 64), 1, 1, 2, 1};
   sp.cm = std::min<int64_t>(32, M), sp.cn = std::min<int64_t>(32, N);

@@ -196,7 +196,8 @@ typedef struct hxm_plan {
  * / F32 otherwise; b_layout as the call's (HXM_B_KN costs a pack
  * workspace); cfg NULL or zeroed = the library's choice (tuned winner, else
  * the default), else that config.  Operands are taken densely packed
- * (lda = ldb = K).  Fills *out (also for a refusal: plan
+ * (lda = ldb = K) and C as overwritten (an accumulating call may take another
+ * default tile; hxm_last_plan tells).  Fills *out (also for a refusal: plan
  * HXM_PLAN_REFUSED and the reason) and returns the status the call would
  * return. */
 hxm_status hxm_plan_matmul(int64_t M, int64_t N, int64_t K, int32_t a_dtype,
