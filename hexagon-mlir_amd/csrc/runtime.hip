@@ -105,6 +105,17 @@ bool stream_capturing(hipStream_t stream) {
   return e != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
+namespace {
+// While it lives, this thread's allocations leave other streams' captures alone:
+// in the default (global) mode a hipMalloc or hipFree of any thread invalidates
+// every capture under way.
+struct RelaxedCaptureMode {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCaptureMode() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCaptureMode() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+}  // namespace
+
 hxm_status stream_workspace(hipStream_t stream, size_t bytes, void** out, int slot, bool* grown) {
   int dev = 0;
   if (grown) *grown = false;
@@ -129,6 +140,7 @@ hxm_status stream_workspace(hipStream_t stream, size_t bytes, void** out, int sl
                   "is kept), or use hxm_gemm_i8_noalloc",
                   w.bytes, bytes);
     size_t grow = bytes < (size_t(1) << 20) ? (size_t(1) << 20) : bytes;
+    const RelaxedCaptureMode relaxed;
     if (w.ptr && w.captured) {
       // A graph holds the old buffer: it stays until hxm_release_cache().
       // Doubling bounds what such buffers add up to by the newest one's size.

@@ -34,7 +34,8 @@
  *     to the output dtype; int8 products accumulate exactly in int32.
  *   - host threads: entries may run at the same time on several host
  *     threads when each uses its own stream (workspaces are per stream; the
- *     device table, the tuning cache and the resident images are locked).
+ *     device table, the tuning cache and the resident images are locked; a
+ *     workspace that grows leaves captures under way on other streams valid).
  *     Calls on one stream must not overlap in time: a call may launch
  *     several kernels that share that stream's workspace, and another
  *     thread's launches in between would reuse it.  hxm_release_cache must

@@ -2,6 +2,8 @@
 one slice to more slices than stages fill, rows and channels that end inside a
 tile and a four-column run, output rows off every alignment; the untuned choice
 of it; and its planes under graph capture."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -157,3 +159,47 @@ def test_requested_split_in_a_graph(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want), rep
+
+
+def test_planes_grow_beside_a_capture(dev):
+    """An untuned call that takes its planes for the first time, then one that
+    has to grow them, on another thread and stream while a graph is captured:
+    the capture stays valid."""
+    g, x, (W,), (s,) = operands(57, 1024, 8192)
+    xs = [x.to(dev), torch.randn(200, 8192, generator=g).half().to(dev)]
+    W, s = W.to(dev), s.to(dev)
+    ys = [torch.empty(xi.shape[0], 1024, dtype=torch.float16, device=dev) for xi in xs]
+    a = torch.randn(64, 4096, generator=g).half().to(dev)
+    o = torch.empty_like(a)
+    ops.softmax(a, out=o)
+    torch.cuda.synchronize()
+    want = o.clone()
+    other, stream, plans, errors = torch.cuda.Stream(), torch.cuda.Stream(), [], []
+    hxm.lib.hxm_release_cache()                      # no planes on any stream
+
+    def work():
+        try:
+            for xi, yi in zip(xs, ys):
+                ops.gemm_w8a16(xi, W, s, out=yi, stream=other)
+                plans.append(ops.last_plan())
+        except Exception as e:                       # reported by the main thread
+            errors.append(e)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        ops.softmax(a, out=o)
+    assert not errors
+    assert all(p["config"][6] > 1 for p in plans)
+    assert plans[1]["workspace_bytes"] > max(plans[0]["workspace_bytes"], 1 << 20)
+    for xi, yi in zip(xs, ys):
+        ref = orc.f16_bits_to_f32(orc.gemm_w8a16(bits(xi), W.cpu().numpy(), s.cpu().numpy()))
+        np.testing.assert_allclose(yi.float().cpu().numpy(), ref, **TOL)
+    for rep in range(3):
+        o.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want), rep
