@@ -352,7 +352,7 @@ hxm_status plan_gemm(int32_t op, int32_t table, int epi, int32_t b_layout, int64
       p->config = small_gemm_config();
       p->threads = 64;
       p->tiles = ((M + 15) / 16) * ((N + 15) / 16);
-      p->lds_bytes = 0;
+      p->lds_bytes = small_gemm_lds(K, b_layout == HXM_B_KN && small_takes_kn(N));
       p->workspace_bytes = extra_ws + (b_layout == HXM_B_KN ? N * kn_image_ld(K, eb) * eb : 0);
       p->k_slices = 1;
       // The plan's classes use the 32-wide MFMA edge for every kernel (the

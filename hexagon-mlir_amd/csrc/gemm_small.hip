@@ -8,7 +8,7 @@
 // fragments straight from memory into registers -- every k-step's A row
 // chunk and B column chunk (16 bytes per lane) issued at once, one round
 // trip -- then runs its v_mfma_f32_16x16x32 chain on two accumulators and
-// stores.  No LDS, no barrier.  Measured in a HIP graph of 50 launches (one
+// stores.  No LDS (a [K, N] B apart, below), no barrier.  Measured in a HIP graph of 50 launches (one
 // box): 256^3 2.20 against 3.19 us for the staged kernel's 32x32 tiles,
 // 128^3 2.03 against 2.77, 300x260x200 2.29 against 3.38; at 512x512x256
 // (1024 tiles) 3.66 against 3.55 and beyond that the staged kernel's
@@ -60,6 +60,7 @@ __device__ __forceinline__ v4f32 mfma16(v4i32 a, v4i32 b, v4f32 c) {
 // picks its fragments out of the words of neighbouring rows, which takes the
 // place of a pack launch before this one (2.6 us of a 256^3 matmul in a HIP
 // graph; called one by one, 13.6 us with the pack, 7.8 without).
+constexpr int kKnPitch = 36;  // bytes per K row in LDS: 16 columns and a word
 template <typename T, int KS, typename OUT, bool ACC, bool KN>
 __global__ __launch_bounds__(64) void small_gemm_kernel(SmallArgs g) {
   const int lane = threadIdx.x;
@@ -71,8 +72,7 @@ __global__ __launch_bounds__(64) void small_gemm_kernel(SmallArgs g) {
   v4i32 av[KS], bv[KS];
   const v4i32 zero = {0, 0, 0, 0};
   if constexpr (KN) {
-    constexpr int kPitch = 36;  // bytes per K row in LDS: 16 columns and a word
-    __shared__ __attribute__((aligned(16))) uint8_t tile[KS * 32 * kPitch];
+    __shared__ __attribute__((aligned(16))) uint8_t tile[KS * 32 * kKnPitch];
     const int half = lane & 1;
     // The last chunk of a row is its last 16 bytes, shifted down.
     const int at = min(n0 + half * 8, g.N - 8), out = min(n0 + half * 8 - at, 8);
@@ -97,13 +97,13 @@ __global__ __launch_bounds__(64) void small_gemm_kernel(SmallArgs g) {
       const v4u32_t o = __builtin_bit_cast(v4u32_t, v);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        *reinterpret_cast<uint32_t*>(tile + k * kPitch + half * 16 + e * 4) = o[e];
+        *reinterpret_cast<uint32_t*>(tile + k * kKnPitch + half * 16 + e * 4) = o[e];
     }
     // One wave: its LDS operations complete in order, and the compiler keeps
     // them so.
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int s = 0; s < KS; ++s) bv[s] = kn_fragment<2>(tile, kPitch, s * 32 + kq * 8, r * 2);
+    for (int s = 0; s < KS; ++s) bv[s] = kn_fragment<2>(tile, kKnPitch, s * 32 + kq * 8, r * 2);
   } else {
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -148,14 +148,18 @@ void launch_ks(const SmallArgs& g, dim3 grid, hipStream_t s) {
                  : small_gemm_kernel<T, KS, __bf16, false, KN><<<grid, 64, 0, s>>>(g);
 }
 
+// Compiled k-steps (32 wide) that hold K.
+int k_steps(int64_t K) { return K <= 32 ? 1 : K <= 64 ? 2 : K <= 128 ? 4 : 8; }
+
 template <typename T, bool KN>
 hxm_status launch_t(const SmallArgs& g, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>((g.N + 15) / 16), static_cast<unsigned>((g.M + 15) / 16));
-  const int ks = (g.K + 31) / 32;
-  if (ks <= 1) launch_ks<T, 1, KN>(g, grid, s);
-  else if (ks <= 2) launch_ks<T, 2, KN>(g, grid, s);
-  else if (ks <= 4) launch_ks<T, 4, KN>(g, grid, s);
-  else launch_ks<T, 8, KN>(g, grid, s);
+  switch (k_steps(g.K)) {
+    case 1: launch_ks<T, 1, KN>(g, grid, s); break;
+    case 2: launch_ks<T, 2, KN>(g, grid, s); break;
+    case 4: launch_ks<T, 4, KN>(g, grid, s); break;
+    default: launch_ks<T, 8, KN>(g, grid, s);
+  }
   return check_launch("small gemm");
 }
 
@@ -173,6 +177,8 @@ bool small_gemm_fits(int64_t M, int64_t N, int64_t K, int32_t ab_dtype) {
   return (ab_dtype == HXM_F16 || ab_dtype == HXM_BF16) && K > 0 && K <= kSmallKMax &&
          M > 0 && N > 0 && ((M + 15) / 16) * ((N + 15) / 16) <= kSmallTilesMax;
 }
+
+int64_t small_gemm_lds(int64_t K, bool kn) { return kn ? k_steps(K) * 32 * kKnPitch : 0; }
 
 hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const uint8_t* B,
                              int64_t ldb_bytes, bool kn, void* C, int64_t ldc, int64_t M,

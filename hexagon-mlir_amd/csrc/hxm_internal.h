@@ -89,6 +89,7 @@ constexpr int64_t kSmallKMax = 256;
 hxm_gemm_config small_gemm_config();
 bool is_small_gemm_config(const hxm_gemm_config& c);
 bool small_gemm_fits(int64_t M, int64_t N, int64_t K, int32_t ab_dtype);
+int64_t small_gemm_lds(int64_t K, bool kn);
 hxm_status launch_small_gemm(int32_t ab_dtype, const void* A, int64_t lda, const uint8_t* B,
                              int64_t ldb_bytes, bool kn, void* C, int64_t ldc, int64_t M,
                              int64_t N, int64_t K, int32_t out_dtype, int32_t accumulate,

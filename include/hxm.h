@@ -227,7 +227,8 @@ int32_t hxm_last_plan(hxm_plan* out);
  * otherwise): the kernels address a tile's rows with 32-bit offsets.
  * With cfg NULL and no tuned winner, an output of at most 512 16x16 tiles
  * with K <= 256 runs on the direct-load small-output kernel (config
- * {16,16,32,1,1,0,1}, one wave per 16x16 tile, no LDS); the same config
+ * {16,16,32,1,1,0,1}, one wave per 16x16 tile, LDS only for a [K,N] B that it reads
+ * as it is, of 8 columns or more); the same config
  * passed in cfg asks for it and is refused (HXM_UNSUPPORTED_SHAPE,
  * "no-kernel") outside those limits.  Other outputs of few rows run on the
  * skinny kernel of the W8A16 GEMMs (config {16,16,64,1,8,0,1}, 1 to 256 rows),

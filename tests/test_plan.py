@@ -128,6 +128,11 @@ def test_small_outputs_plan_the_direct_kernel():
     assert plan(256, 256, 256, I8)["config"] != small
     kn = plan(128, 128, 128, F16, b_layout="kn")
     assert kn["config"] == small and kn["workspace_bytes"] == 128 * 128 * 2
+    # [K, N] rows of 16 columns and a word in LDS, 32 of them a compiled k-step;
+    # fewer than 8 columns are packed first.
+    for K, steps in ((8, 1), (64, 2), (72, 4), (256, 8)):
+        assert plan(64, 8, K, BF16, b_layout="kn")["lds_bytes"] == steps * 32 * 36
+        assert plan(64, 7, K, BF16, b_layout="kn")["lds_bytes"] == 0
     named = plan(64, 64, 64, F16, config=small)
     assert named["config"] == small and named["source"] == "caller"
     refused = plan(1024, 1024, 1024, F16, config=small)
