@@ -77,7 +77,9 @@ const KernelEntry* find_kernel(const hxm_gemm_config& c, int32_t dt) {
 // prologue, epilogue) plus its K stages of 128 bytes; a stage costs stage_lo
 // on an otherwise idle chip (latency, issue) and stage_hi on a full one (L2 ->
 // LDS bandwidth, clock).  int8 and f16/bf16 stages of the same bytes take the
-// same time.  Fitted to tuner measurements (us, one box; modeled / measured):
+// same time.  Fitted by hand to tuner measurements, seven of them here; it ranks
+// the tiles and is no forecast (1500 x 2047 x 512 takes 12.7 us on its choice,
+// 11.1 on the four-stage 64x64) (us, one box; modeled / measured):
 //   f16 512 x 4096 x 4096: 128x64 26 / 23.8, 64x64 31 / 28.6, 128x128 36 / 26.9
 //     (two-stage 64x64, the default before: 35.3)
 //   bf16 1776 x 1640 x 4448: 128x128 41 / 40.1, 128x64 51 / 56 (before: 52.0)
@@ -94,7 +96,9 @@ const KernelEntry* find_kernel(const hxm_gemm_config& c, int32_t dt) {
 // store: bf16 2772 x 4091 x 192 256x256 35.8, 256x128 27.9, 128x128 21.9, 64x64
 // 21.1, 128x128 of two stages (two workgroups a CU) 18.4.  The last is offered
 // for such an N only, where two fit and K is at most 16 stages (1024: 36.0 us
-// against 38.1; 2048: 59.2 against 57.8).
+// against 38.1; 2048: 59.2 against 57.8).  On the boundary it is not, though a
+// short K would gain there too (f16 2772 x 4096 x 192 13.2 us, 11.7 with it;
+// 4096 x 4096 x 256 17.0, 19.1): the constants were fitted without it.
 //
 // An accumulating call takes the general epilogue at every N and reads each run
 // of C before it can store it (`rmw` more a workgroup).  What hides that wait is

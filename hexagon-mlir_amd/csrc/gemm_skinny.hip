@@ -1,6 +1,7 @@
 // Launch rules of the skinny matmuls (skinny_kernel.h): the default of the
 // W8A16 GEMMs, of hxm_gemm_i8 / _dequant and of hxm_matmul at 1 to
-// kSkinnyRowsMax rows, and of hxm_gemv_w8a16 on plain [N, K] weights at 2 to 16.
+// kSkinnyRowsMax rows, and of hxm_gemv_w8a16 on plain [N, K] weights at any M > 1
+// (in blocks of 16 rows, one grid row each).
 #include "skinny_kernel.h"
 
 namespace hxm {

@@ -423,8 +423,9 @@ __global__ __launch_bounds__(row_waves(S) * 64) void row_kernel(RowArgs a) {
 // columns, then this kernel with S = 1): the mean of a long row is the
 // difference of near-equal sums, and its fp32 rounding in another order (a few
 // 1e-6 of a mean near zero at 1e5 columns) would show in the mean and rstd
-// that callers keep for the backward pass.  Eight loads in flight: 175 x 50688
-// 229 -> 88 us, 4096 x 8192 (registers) 75.7 -> 47.3.
+// that callers keep for the backward pass.  (Compensated or 64-bit partial sums
+// over more waves would be nearer the true mean; not built.)  Eight loads in
+// flight: 175 x 50688 229 -> 88 us, 4096 x 8192 (registers) 75.7 -> 47.3.
 template <typename T, int OP, int S>
 __global__ __launch_bounds__(S * 64) void row_kernel_stream(RowArgs a) {
   constexpr int N = RowVec<T>::N;

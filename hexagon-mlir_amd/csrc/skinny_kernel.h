@@ -1,6 +1,7 @@
 #pragma once
-// Skinny MFMA matmuls on gfx950: up to 64 rows of A per workgroup (a call has
-// at most kSkinnyRowsMax) against the [N, K] image of B, or B as it is [K, N].
+// Skinny MFMA matmuls on gfx950: up to 64 rows of A per workgroup (a GEMM or
+// matmul has at most kSkinnyRowsMax; the plain-layout GEMV any number, 16 at a
+// time) against the [N, K] image of B, or B as it is [K, N].
 //
 // What bounds such a call is the weight stream: each weight byte meets at
 // most 64 rows, far below the matrix cores' ratio.  The LDS-staged tiles

@@ -164,7 +164,9 @@ def test_float(dev, dt, M, N, K):
     np.testing.assert_allclose(h.float().cpu().numpy(), ref, rtol=1e-2, atol=1e-3)
 
 
-@pytest.mark.parametrize("M", [2, 4, 5, 16, 17, 40])
+# The GEMV takes any number of rows, 16 at a time: 261 and 300 end in partial blocks
+# past the row limit of the GEMMs.
+@pytest.mark.parametrize("M", [2, 4, 5, 16, 17, 40, 261, 300])
 @pytest.mark.parametrize("N,K", [(40, 16), (333, 656), (100, 2064)])
 def test_gemv_plain_weights(dev, M, N, K):
     print(f"skinny gemv M={M} N={N} K={K}", flush=True)
